@@ -1475,78 +1475,154 @@ constexpr int kHotDN = 128;        // bags per dot-product tile
 constexpr int kHotDK = 64;         // dims per chunk of the dot product
 constexpr int kHotThreads = 256;   // 4 waves of 64 x 64
 constexpr uint32_t kHotLo = 0x80000000u;  // chunk-pointer flag: the row's chunk holds a lo entry
-constexpr int kHotLoList = 256;    // lo chunks one row lists before it flags all of its chunks
 
-// For each listed row i (row r = hot[i], count at hot[hr_max]; sorted
-// occurrences [offs[r], offs[r+1])): the row's entries, one per distinct bag
-// in bag order, written over the start of the row's own occurrence range of
-// ent (bag % 32 | hi << 16) and ent_lo (lo); chunk pointers, chunk-major
-// (index c * hr_max + i), pc (first entry, | kHotLo if the chunk holds a lo)
-// and po (first occurrence) of the row's first bag >= 32 c, for c = 0..nc (c =
-// nc: the row's ends); any_lo <- 1 if some lo is nonzero. A block per row,
-// grid-stride over the list (every block reads the count).
-__global__ __launch_bounds__(256) void hot_list_kernel(const uint32_t* __restrict__ hot, int64_t hr_max,
-                                                       const uint32_t* __restrict__ offs,
-                                                       const uint2* __restrict__ meta, uint32_t nc,
-                                                       uint32_t* __restrict__ pc, uint32_t* __restrict__ po,
-                                                       uint32_t* __restrict__ ent, uint16_t* __restrict__ ent_lo,
-                                                       uint32_t* __restrict__ any_lo) {
-  __shared__ uint32_t lds4[4];
-  __shared__ uint32_t lo_chunks[kHotLoList];
-  __shared__ uint32_t n_lo;
+// The hot rows' chunk pointers and entries, by occurrence (every lookup of a
+// hot row is one thread's, whatever its row's length): a row with 10^5
+// lookups is spread over as many waves as 10^5 lookups of short rows. A block
+// per row (256 lookups a step, two barriers and a serial walk of each bag's
+// run of lookups per step) took 3.86 ms for 2 M Zipf(1.1) lookups of 8192 bags
+// (one row holding a tenth of them); the two kernels below take 0.05 ms.
+//
+// hot_slot: the list position of occurrence j's row, or -1 where the row is
+// not hot. The list is in row order; a wave inside one row (most of them)
+// searches it once, with uniform loads.
+__device__ __forceinline__ int hot_slot(uint32_t r, bool valid, const uint32_t* __restrict__ hot, uint32_t n,
+                                        const uint32_t* __restrict__ offs, uint32_t H, uint32_t* beg, uint32_t* end) {
+  const uint32_t r0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)r);
+  const bool uniform = __ballot(valid && r == r0) == ~0ull;
+  if (uniform) {
+    *beg = offs[r0];
+    *end = offs[r0 + 1];
+    if (*end - *beg < H) return -1;
+    uint32_t lo = 0, hi = n;
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (hot[mid] < r0)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    return (int)lo;
+  }
+  if (!valid) return -1;
+  *beg = offs[r];
+  *end = offs[r + 1];
+  if (*end - *beg < H) return -1;
+  uint32_t lo = 0, hi = n;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (hot[mid] < r)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  return (int)lo;
+}
+
+// Chunk pointers, chunk-major (index c * hr_max + i): pc and po of (chunk c,
+// list position i) = the first sorted occurrence of the row hot[i] in a bag >=
+// 32 c, for c = 0..nc (c = nc: the row's end). hot_entries_kernel flags pc.
+__global__ __launch_bounds__(256) void hot_chunks_kernel(const uint32_t* __restrict__ hot, int64_t hr_max,
+                                                         const uint32_t* __restrict__ offs,
+                                                         const uint32_t* __restrict__ skeys,
+                                                         const uint32_t* __restrict__ nvalid,
+                                                         const uint2* __restrict__ meta, uint32_t hot_min, uint32_t nc,
+                                                         uint32_t* __restrict__ pc, uint32_t* __restrict__ po) {
   const uint32_t n = hot[hr_max];
+  if (n == 0) return;
+  const uint32_t nv = *nvalid;
   const size_t H = (size_t)hr_max;
-  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-    const uint32_t r = hot[i];
-    const uint32_t beg = offs[r], end = offs[r + 1];
-    if (threadIdx.x == 0) n_lo = 0u;
-    __syncthreads();
-    uint32_t carry = 0;  // entries of the row's earlier occurrence tiles
-    for (uint32_t j0 = beg; j0 < end; j0 += 256) {
-      const uint32_t j = j0 + threadIdx.x;
-      uint32_t bag = 0, prev = 0;
-      bool start = false;
-      if (j < end) {
-        bag = meta[j].x;
-        prev = j > beg ? meta[j - 1].x : 0u;
-        start = j == beg || bag != prev;
-      }
-      uint32_t tot;
-      const uint32_t k = carry + block_exclusive_sum(start ? 1u : 0u, &tot, lds4);
-      if (start) {
-        // chunks (chunk of the previous occurrence, chunk of this one] start here
-        const uint32_t c = bag / kHotKC;
-        for (uint32_t cc = j == beg ? 0u : prev / kHotKC + 1u; cc <= c; ++cc) {
-          pc[cc * H + i] = beg + k;
-          po[cc * H + i] = j;
-        }
-        float s = __uint_as_float(meta[j].y);
-        for (uint32_t t = j + 1; t < end && meta[t].x == bag; ++t) s += __uint_as_float(meta[t].y);
-        const uint32_t hi = f32_to_bf16_bits(s);
-        const uint32_t lo = f32_to_bf16_bits(s - bf16_to_f32(hi));
-        ent[beg + k] = (bag % kHotKC) | (hi << 16);
-        ent_lo[beg + k] = (uint16_t)lo;
-        if ((lo & 0x7FFFu) != 0u) {
-          *any_lo = 1u;
-          const uint32_t at = atomicAdd(&n_lo, 1u);
-          if (at < (uint32_t)kHotLoList) lo_chunks[at] = c;
-        }
-      }
-      carry += tot;
+  for (uint32_t j0 = blockIdx.x * 256; j0 < nv; j0 += gridDim.x * 256) {
+    const uint32_t j = j0 + threadIdx.x;
+    const bool valid = j < nv;
+    uint32_t beg = 0, end = 0;
+    const int i = hot_slot(valid ? skeys[j] : 0u, valid, hot, n, offs, hot_min, &beg, &end);
+    if (i < 0) continue;
+    // chunks (chunk of the row's previous occurrence, chunk of this one] start here
+    const uint32_t c = meta[j].x / kHotKC;
+    for (uint32_t cc = j == beg ? 0u : meta[j - 1].x / kHotKC + 1u; cc <= c; ++cc) {
+      pc[cc * H + i] = j;
+      po[cc * H + i] = j;
     }
-    const uint32_t c_end = end > beg ? meta[end - 1].x / kHotKC + 1u : 0u;
-    for (uint32_t cc = c_end + threadIdx.x; cc <= nc; cc += 256) {
-      pc[cc * H + i] = beg + carry;
-      po[cc * H + i] = end;
+    if (j + 1 == end)
+      for (uint32_t cc = c + 1; cc <= nc; ++cc) {
+        pc[cc * H + i] = end;
+        po[cc * H + i] = end;
+      }
+  }
+}
+
+// The merged entries of each (hot row, chunk), at the chunk's own occurrences
+// of ent (bag % 32 | hi << 16) and ent_lo (lo); the first min(32, occurrences)
+// of them are read. A chunk of fewer than 32 occurrences holds at each
+// occurrence the entry of its bag (a bag read twice: the same entry twice);
+// one of 32 or more holds bag 32 c + s's entry at s, of weight zero where the
+// row has no lookup in the bag. Either way the place of an entry needs no
+// count of the entries before it. Flags the pc of a chunk that holds a lo
+// entry; any_lo <- 1 if some lo is nonzero.
+__global__ __launch_bounds__(256) void hot_entries_kernel(
+    const uint32_t* __restrict__ hot, int64_t hr_max, const uint32_t* __restrict__ offs,
+    const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ nvalid, const uint2* __restrict__ meta,
+    uint32_t hot_min, uint32_t* __restrict__ pc, const uint32_t* __restrict__ po, uint32_t* __restrict__ ent,
+    uint16_t* __restrict__ ent_lo, uint32_t* __restrict__ any_lo) {
+  const uint32_t n = hot[hr_max];
+  if (n == 0) return;
+  const uint32_t nv = *nvalid;
+  const size_t H = (size_t)hr_max;
+  for (uint32_t j0 = blockIdx.x * 256; j0 < nv; j0 += gridDim.x * 256) {
+    const uint32_t j = j0 + threadIdx.x;
+    const bool valid = j < nv;
+    uint32_t beg = 0, end = 0;
+    const int i = hot_slot(valid ? skeys[j] : 0u, valid, hot, n, offs, hot_min, &beg, &end);
+    if (i < 0) continue;
+    const uint2 m = meta[j];
+    const uint32_t prev = j > beg ? meta[j - 1].x : 0u;
+    if (j > beg && m.x == prev) continue;  // its bag's first occurrence writes the entry
+    const uint32_t c = m.x / kHotKC;
+    const uint32_t s = po[c * H + i], e = po[(c + 1) * H + i];
+    // the bag's weights in position order; 8 occurrences a step (meta is padded past its end)
+    float w = __uint_as_float(m.y);
+    uint32_t t = j + 1;
+    for (bool more = true; more && t < e;) {
+      uint2 x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = meta[t + u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        more = more && t < e && x[u].x == m.x;
+        if (more) {
+          w += __uint_as_float(x[u].y);
+          ++t;
+        }
+      }
     }
-    __syncthreads();  // every pointer of the row written, n_lo final
-    const uint32_t nl = n_lo;
-    if (nl > (uint32_t)kHotLoList) {
-      for (uint32_t cc = threadIdx.x; cc < nc; cc += 256) pc[cc * H + i] |= kHotLo;
+    const uint32_t hi = f32_to_bf16_bits(w);
+    const uint16_t lo = (uint16_t)f32_to_bf16_bits(w - bf16_to_f32(hi));
+    const uint32_t slot = m.x % kHotKC;
+    const uint32_t entry = slot | (hi << 16);
+    if (e - s >= (uint32_t)kHotKC) {
+      ent[s + slot] = entry;
+      ent_lo[s + slot] = lo;
+      // the empty bags before this one, and after the chunk's last
+      for (uint32_t z = j == s ? 0u : prev % kHotKC + 1u; z < slot; ++z) {
+        ent[s + z] = z;
+        ent_lo[s + z] = 0;
+      }
+      if (t == e)
+        for (uint32_t z = slot + 1; z < (uint32_t)kHotKC; ++z) {
+          ent[s + z] = z;
+          ent_lo[s + z] = 0;
+        }
     } else {
-      for (uint32_t t = threadIdx.x; t < nl; t += 256) atomicOr(&pc[lo_chunks[t] * H + i], kHotLo);
+      for (uint32_t z = j; z < t; ++z) {
+        ent[z] = entry;
+        ent_lo[z] = lo;
+      }
     }
-    __syncthreads();  // n_lo and lo_chunks before the next row
+    if ((lo & 0x7FFFu) != 0u) {
+      pc[c * H + i] = s | kHotLo;  // (every bag of the chunk that has one writes the same word)
+      *any_lo = 1u;
+    }
   }
 }
 
@@ -2285,7 +2361,7 @@ static void launch_rows_dyn(const void* W, int64_t K, int64_t D, int want_dot, c
 // row and the row kernel's lists.
 template <typename TW, int LPG, int VPL>
 static void launch_prepare(int64_t K, int64_t D, const void* psw, int pdt, int64_t L, const uint32_t* offs,
-                           const uint32_t* svals, const uint32_t* nvalid, int64_t N, const BwdLayout& l, char* ws,
+                           const uint32_t* skeys, const uint32_t* svals, const uint32_t* nvalid, int64_t N, const BwdLayout& l, char* ws,
                            bool hot, hipStream_t st) {
   if constexpr (LPG == 64) {
     uint2* meta = (uint2*)(ws + l.meta);
@@ -2302,13 +2378,17 @@ static void launch_prepare(int64_t K, int64_t D, const void* psw, int pdt, int64
       prepare_rows_dyn(K, rows_prefetch<VPL>(N, K), offs, (uint32_t*)(ws + l.long_rows), st);
     if constexpr (std::is_same<TW, bf16_t>::value) {
       if (hot && hot_rows_enabled(l, D)) {
-        // the hot rows the sort listed: merged entries and chunk pointers
+        // the hot rows the sort listed: chunk pointers and merged entries (blocks past the list's need end at once)
         const uint32_t* hot_list = (const uint32_t*)(ws + l.hot_rows);
-        const unsigned gb = (unsigned)(l.hr_max < 8192 ? l.hr_max : 8192);  // a block per row, up to 8192
-        hipLaunchKernelGGL(hot_list_kernel, dim3(gb), dim3(256), 0, st, hot_list, l.hr_max, offs,
-                           (const uint2*)(ws + l.meta), (uint32_t)l.hot_nc, (uint32_t*)(ws + l.hot_pc),
-                           (uint32_t*)(ws + l.hot_po), (uint32_t*)(ws + l.hot_ent), (uint16_t*)(ws + l.hot_lo),
-                           (uint32_t*)(ws + l.hot_rows) + l.hr_max + 1);
+        const uint2* m = (const uint2*)(ws + l.meta);
+        uint32_t* pc = (uint32_t*)(ws + l.hot_pc);
+        uint32_t* po = (uint32_t*)(ws + l.hot_po);
+        const dim3 gb(grid_for(N, 256, 4096));
+        hipLaunchKernelGGL(hot_chunks_kernel, gb, dim3(256), 0, st, hot_list, l.hr_max, offs, skeys, nvalid, m,
+                           (uint32_t)l.hot_min, (uint32_t)l.hot_nc, pc, po);
+        hipLaunchKernelGGL(hot_entries_kernel, gb, dim3(256), 0, st, hot_list, l.hr_max, offs, skeys, nvalid, m,
+                           (uint32_t)l.hot_min, pc, (const uint32_t*)po, (uint32_t*)(ws + l.hot_ent),
+                           (uint16_t*)(ws + l.hot_lo), (uint32_t*)(ws + l.hot_rows) + l.hr_max + 1);
       }
     }
   }
@@ -2416,7 +2496,7 @@ static bool dispatch_reduce(bool prepare, const GroupCfg& c, const void* W, int6
 #define PKM_RED_CASE(LPG_, VPL_)                                                                                  \
   if (c.lpg == LPG_ && c.vpl == VPL_) {                                                                           \
     if (prepare) {                                                                                                \
-      launch_prepare<TW, LPG_, VPL_>(K, D, psw, pdt, L, offs, svals, nvalid, N, l, ws, hot, st);                  \
+      launch_prepare<TW, LPG_, VPL_>(K, D, psw, pdt, L, offs, skeys, svals, nvalid, N, l, ws, hot, st);           \
     } else if (sgd == nullptr && acc) {                                                                         \
       if constexpr (LPG_ == 64 && std::is_same<TW, TG>::value)                                                    \
         launch_reduce<TW, TG, LPG_, VPL_, false, true>(W, K, D, psw, pdt, g, L, offs, skeys, svals, nvalid, N, l, \

@@ -539,6 +539,36 @@ def test_backward_hot_rows_merged_weights_exact(D, psw_dtype, device):
     assert_rel_close(gp, ep, 1e-4 if psw_dtype == torch.float32 else REL_TOL[psw_dtype], "grad_psw", cond=cp)
 
 
+# Hot rows whose 32-bag chunks hold fewer than 32 lookups, exactly 31, 32 and
+# 33, and many more (a bag holding a row up to L times: a run that spans waves),
+# with bags in between that do not hold the row, and a last chunk of 28 bags.
+# Tolerances as above: one bf16 rounding of sums taken in another order.
+@pytest.mark.parametrize("L", [48, 200])
+def test_backward_hot_rows_chunk_densities(L, device):
+    from modelos_amd import embedding_bag as eb
+
+    B, K, D = 700, 3000, 512
+    W, _, p, g = eb_inputs(B, L, K, D, torch.bfloat16, seed=71 + L)
+    gen = torch.Generator().manual_seed(72 + L)
+    idx = torch.randint(20, K, (B, L), generator=gen)
+    bag = torch.arange(B)
+    idx[:, 0] = 5  # 32 a chunk
+    idx[bag % 32 != 7, 1] = 6  # 31, the empty bag inside
+    idx[:, 2] = 7
+    idx[bag % 32 == 31, 3] = 7  # 33, the chunk's last bag twice
+    idx[bag % 2 == 1, 4] = 8  # 16, every other bag
+    for b in range(B):  # 0 to L - 8 lookups of row 9
+        idx[b, 8:8 + (b * 37) % (L - 7)] = 9
+    idx[100:130, 8:] = 9  # whole bags of one row
+    gW, gp = eb.eb_backward(*_dev(idx, W, p, g, device=device))
+    eW, ep = ref.eb_backward(idx, W, p, g)
+    cW, cp = ref.eb_backward(idx, W.abs(), p.abs(), g.abs())
+    assert_rel_close(gW, eW, REL_TOL[torch.bfloat16], "grad_weight", cond=cW)
+    assert_rel_close(gp, ep, REL_TOL[torch.bfloat16], "grad_psw", cond=cp)
+    gW2, gp2 = eb.eb_backward(*_dev(idx, W, p, g, device=device))
+    assert torch.equal(gW, gW2) and torch.equal(gp, gp2)
+
+
 # Rows longer than the row kernel's prefetch but below the heavy threshold
 # (5..250 lookups), packed into the first 64-row windows, beside two heavy rows
 # and uniform rows: with more than 3 lookups per row on average (the 8-slot
