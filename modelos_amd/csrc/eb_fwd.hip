@@ -7,8 +7,9 @@
 // increasing order, one rounding to the table dtype at the end (:113, output
 // allocated in weight.dtype at :123).
 //
-// Mapping (HBM-bound gather): a "lane group" of LPG lanes (LPG = 64: one
-// wave) owns one (bag, column-slice) task. Each lane holds VPL 16-byte vectors
+// Mapping of the double backward, and of the forward's rows that are not whole
+// 256-byte pieces (the others run on eb_gather_kernel): a "lane group" of LPG
+// lanes (LPG = 64: one wave) owns one (bag, column-slice) task. Each lane holds VPL 16-byte vectors
 // of the slice, so one row read by the group is LPG*VPL*16 contiguous bytes
 // (2 KB for a bf16 row of 1024 at LPG=64, VPL=2). The group loads LPG bag
 // entries (index + weight) with one coalesced access, broadcasts them lane by
@@ -21,6 +22,8 @@
 // The upstream gradient g and the gathered sum (d_grad_out) are of type TG:
 // the table's type, or float32 beside a 16-bit gbar (read in its own dtype,
 // float32 arithmetic as the reference's type promotion gives).
+#include <utility>
+
 #include "pkm_common.h"
 
 namespace pkm {
@@ -176,6 +179,123 @@ __global__ __launch_bounds__(256) void eb_fwd_kernel(const TW* __restrict__ W, i
   }
 }
 
+// ---------------------------------------------------------------------------
+// The forward gather: a wave owns BPW bags x a slice of 64 / BPW vectors of
+// the row, NW waves share a task's lookups. A gather of rows from a table
+// larger than the Infinity Cache (256 MB) is bound by the lines in flight per
+// CU times their latency. With enough bags to fill the chip with one slice
+// (slices slowest over the grid), a slice of the table at a time is partly
+// answered by that cache: two bags x 512 bytes a wave, 16384 bags into 2^20 x
+// 1024 bf16 (whole 2 KB rows per wave, the kernel this one replaced -> this
+// one): 690 -> 628 us at 128 lookups a bag, 1367 -> 1229 us at 256 (7.0 TB/s);
+// 256-byte slices 635 us, 1 KB slices 648 us, 128-byte slices 670 us. With
+// fewer bags every slice is in flight at once and slicing only scatters the
+// reads: one bag a wave, slices fastest (4096 bags x 128, 2^18 x 512: 77 us,
+// 83 us sliced; 500 x 500, 2^16 x 2048: 142 us, 152 us sliced).
+//
+// Row numbers and weights are held 16 to a register in each 16-lane row and
+// broadcast by DPP; the next 16 are loaded a step ahead. Absent lookups read a
+// line of zeros, with weight zero: no load is conditional.
+//
+// NW > 1 where the tasks alone leave the chip idle: 16 lookups each in turn,
+// the waves' float32 sums added in wave order through LDS (8 bags x 256: one
+// wave's serial chain of 32 loads 42 us, 16 waves' chains of 2 11 us).
+// ---------------------------------------------------------------------------
+constexpr int kGatherLanes = 16;
+constexpr int kGatherMaxNW = 16;
+
+__device__ uint4 g_zero_line[64];
+
+template <int K>
+__device__ __forceinline__ uint32_t row16_bcast(uint32_t v) {  // lane K of each 16-lane row (DPP row_newbcast)
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x150 + K, 0xF, 0xF, false);
+}
+
+// acc += the 8 lookups held by lanes J0 .. J0 + 7 of each 16-lane row, in order
+template <typename TW, int J0, int... I>
+__device__ __forceinline__ void gather8(const char* base, uint64_t row_bytes, uint32_t r, float w, const char* zero,
+                                        float* acc, std::integer_sequence<int, I...>) {
+  constexpr int EPV = VecTraits<TW>::EPV;
+  uint4 v[8];
+  ((v[I] = [&] {
+     const uint32_t rr = row16_bcast<J0 + I>(r);
+     return ld16(rr != 0xFFFFFFFFu ? base + (uint64_t)rr * row_bytes : zero);
+   }()),
+   ...);
+  ([&] {
+    const float ww = __uint_as_float(row16_bcast<J0 + I>(__float_as_uint(w)));
+    float f[EPV];
+    VecTraits<TW>::unpack(v[I], f);
+#pragma unroll
+    for (int e = 0; e < EPV; ++e) acc[e] = __builtin_fmaf(f[e], ww, acc[e]);
+  }(),
+   ...);
+}
+
+template <typename TW, int BPW>
+__global__ __launch_bounds__(64 * kGatherMaxNW) void eb_gather_kernel(const TW* __restrict__ W, int64_t K, int64_t D,
+                                                                      const int64_t* __restrict__ idx,
+                                                                      const void* __restrict__ psw, int pdt,
+                                                                      int64_t B, int64_t L, int64_t S, int NW,
+                                                                      TW* __restrict__ out) {
+  constexpr int EPV = VecTraits<TW>::EPV;
+  extern __shared__ __align__(16) float gather_part[];  // NW > 1: [wave][lane][EPV]
+  constexpr int SL = 64 / BPW;  // lanes (vectors) per slice
+  const int lane = threadIdx.x & 63, gl = lane & (kGatherLanes - 1);
+  const int wave = threadIdx.x >> 6;
+  const int q = wave & (NW - 1);  // this wave's share of its task's lookups
+  const int64_t groups = (B + BPW - 1) / BPW;
+  const int64_t task = ((int64_t)blockIdx.x * (blockDim.x >> 6) + wave) / NW;
+  const int64_t s = BPW == 1 ? task % S : task / groups;
+  const int64_t b = BPW == 1 ? task / S : (task - s * groups) * BPW + lane / SL;
+  const bool live = s < S && b < B;
+  const int64_t col0 = (s * SL + (lane & (SL - 1))) * EPV;
+  const char* base = (const char*)(W + col0);
+  const char* zero = (const char*)(g_zero_line + lane);
+  const uint64_t row_bytes = (uint64_t)D * sizeof(TW);
+  const int64_t pb = b * L;
+  const int64_t step = (int64_t)kGatherLanes * NW;
+  float acc[EPV];
+#pragma unroll
+  for (int e = 0; e < EPV; ++e) acc[e] = 0.f;
+  int64_t r_next = -1;
+  float w_next = 0.f;
+  auto fetch = [&](int64_t j0) {
+    r_next = -1;
+    if (live && j0 + gl < L) {
+      r_next = idx[pb + j0 + gl];
+      w_next = psw ? load_scalar(psw, pdt, pb + j0 + gl) : 1.f;
+    }
+  };
+  fetch(kGatherLanes * q);
+  for (int64_t j0 = kGatherLanes * q; j0 < L; j0 += step) {
+    const bool ok = r_next >= 0 && r_next < K;
+    const uint32_t r = ok ? (uint32_t)r_next : 0xFFFFFFFFu;
+    const float w = ok ? w_next : 0.f;
+    fetch(j0 + step);
+    gather8<TW, 0>(base, row_bytes, r, w, zero, acc, std::make_integer_sequence<int, 8>{});
+    gather8<TW, 8>(base, row_bytes, r, w, zero, acc, std::make_integer_sequence<int, 8>{});
+  }
+  if (NW > 1) {
+    float* p = gather_part + (int)threadIdx.x * EPV;
+#pragma unroll
+    for (int e = 0; e < EPV; e += 4) *(float4*)(p + e) = make_float4(acc[e], acc[e + 1], acc[e + 2], acc[e + 3]);
+    __syncthreads();
+    if (q != 0) return;
+    for (int k = 1; k < NW; ++k) {
+#pragma unroll
+      for (int e = 0; e < EPV; e += 4) {
+        const float4 x = *(const float4*)(p + k * 64 * EPV + e);
+        acc[e] += x.x;
+        acc[e + 1] += x.y;
+        acc[e + 2] += x.z;
+        acc[e + 3] += x.w;
+      }
+    }
+  }
+  if (live) st16(out + b * D + col0, VecTraits<TW>::pack(acc));
+}
+
 // Fallback for a row length that is not a multiple of the 16-byte vector:
 // one thread per output element (forward only).
 template <typename TW>
@@ -262,6 +382,41 @@ static void launch_fwd(const void* W, int64_t K, int64_t D, const int64_t* idx, 
                      D, idx, psw, pdt, B, L, S, (TG*)out, (const TG*)g, dot_out, ddt, A);
 }
 
+constexpr int64_t kGatherSliceBags = 8192;  // two bags a wave: half the chip's wave slots from one slice
+constexpr int64_t kGatherFill = 2048;       // waves under which a task's lookups are shared (8 a CU)
+
+template <typename TW, int BPW>
+static void launch_gather(const void* W, int64_t K, int64_t D, const int64_t* idx, const void* psw, int pdt, int64_t B,
+                          int64_t L, void* out, hipStream_t stream) {
+  constexpr int EPV = VecTraits<TW>::EPV;
+  const int64_t S = D / (64 / BPW * EPV);
+  const int64_t tasks = (B + BPW - 1) / BPW * S;
+  int nw = 1;
+  while (nw < kGatherMaxNW && tasks * nw < kGatherFill && L > (int64_t)kGatherLanes * nw) nw *= 2;
+  const int waves = nw > 4 ? nw : 4;
+  KernelSpan span("eb_fwd", stream);
+  hipLaunchKernelGGL((eb_gather_kernel<TW, BPW>), dim3((unsigned)((tasks * nw + waves - 1) / waves)), dim3(64 * waves),
+                     nw > 1 ? (size_t)waves * 64 * EPV * sizeof(float) : 0, stream, (const TW*)W, K, D, idx, psw, pdt,
+                     B, L, S, nw, (TW*)out);
+}
+
+// Rows of whole 16-vector pieces, and row numbers that fit a register (a
+// larger table does not fit the device); false: nothing launched.
+template <typename TW>
+static bool try_gather(const void* W, int64_t K, int64_t D, const int64_t* idx, const void* psw, int pdt, int64_t B,
+                       int64_t L, void* out, hipStream_t stream) {
+  constexpr int EPV = VecTraits<TW>::EPV;
+  if (D % (kGatherLanes * EPV) != 0 || K >= 0xFFFFFFFFll) return false;
+  const int64_t nvec = D / EPV;
+  if (nvec % 64 == 0 && B < kGatherSliceBags)
+    launch_gather<TW, 1>(W, K, D, idx, psw, pdt, B, L, out, stream);
+  else if (nvec % 32 == 0)
+    launch_gather<TW, 2>(W, K, D, idx, psw, pdt, B, L, out, stream);
+  else
+    launch_gather<TW, 4>(W, K, D, idx, psw, pdt, B, L, out, stream);
+  return true;
+}
+
 template <typename TW, bool DOT, typename TG = TW, bool SGDB = false>
 static bool dispatch_fwd(const GroupCfg& c, const void* W, int64_t K, int64_t D, const int64_t* idx,
                          const void* psw, int pdt, int64_t B, int64_t L, void* out, const void* g,
@@ -271,12 +426,14 @@ static bool dispatch_fwd(const GroupCfg& c, const void* W, int64_t K, int64_t D,
     launch_fwd<TW, TG, LPG_, VPL_, DOT, SGDB>(W, K, D, idx, psw, pdt, B, L, c.slices, out, g, dot_out, ddt, A, stream); \
     return true;                                                                                      \
   }
-  PKM_FWD_CASE(64, 1)
-  PKM_FWD_CASE(64, 2)
-  PKM_FWD_CASE(64, 4)
-  PKM_FWD_CASE(64, 8)
-  PKM_FWD_CASE(32, 1)
-  PKM_FWD_CASE(16, 1)
+  if constexpr (DOT) {  // (the forward's rows of whole 16-vector slices go to eb_gather_kernel)
+    PKM_FWD_CASE(64, 1)
+    PKM_FWD_CASE(64, 2)
+    PKM_FWD_CASE(64, 4)
+    PKM_FWD_CASE(64, 8)
+    PKM_FWD_CASE(32, 1)
+    PKM_FWD_CASE(16, 1)
+  }
   PKM_FWD_CASE(8, 1)
   PKM_FWD_CASE(4, 1)
   PKM_FWD_CASE(2, 1)
@@ -310,7 +467,13 @@ extern "C" int pkm_eb_fwd(const void* weight, int64_t num_rows, int64_t dim, int
   GroupCfg c;
   bool ok = false;
   const bool aligned = ((uintptr_t)weight % 16 == 0) && ((uintptr_t)out % 16 == 0);
-  if (aligned && choose_group_cfg(dim, epv_of(weight_dtype), false, &c)) {
+  if (aligned) {
+#define PKM_GATHER(TW_) try_gather<TW_>(weight, num_rows, dim, indices, psw, psw_dtype, bags, bag_size, out, st)
+    ok = weight_dtype == PKM_DTYPE_F32 ? PKM_GATHER(float)
+                                       : (weight_dtype == PKM_DTYPE_BF16 ? PKM_GATHER(bf16_t) : PKM_GATHER(f16_t));
+#undef PKM_GATHER
+  }
+  if (!ok && aligned && choose_group_cfg(dim, epv_of(weight_dtype), false, &c)) {
     if (weight_dtype == PKM_DTYPE_F32)
       ok = dispatch_fwd<float, false>(c, weight, num_rows, dim, indices, psw, psw_dtype, bags, bag_size, out,
                                       nullptr, nullptr, 0, st);

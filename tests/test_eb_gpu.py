@@ -79,6 +79,32 @@ def test_forward_unweighted_mixed_dtypes_and_invalid(device):
     assert eb.count_invalid_indices(didx, 700) == 3
 
 
+# The gather's layouts: whole rows with one to sixteen waves per bag (few bags;
+# bag lengths around the 16-lookup steps), two bags a wave from 8192 bags on
+# (an odd count), rows of 32 k and 16 k vectors. Row 0 holds infinities and is
+# only looked up out of range: absent lookups, with NaN weights, add nothing.
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("B,L,nvec", [(1, 256, 128), (8, 17, 64), (3, 1, 64), (40, 100, 128), (8193, 5, 64),
+                                      (70, 33, 96), (70, 16, 48), (5, 300, 16)])
+def test_forward_gather_layouts(B, L, nvec, dtype, device):
+    from modelos_amd import embedding_bag as eb
+
+    D = nvec * (4 if dtype == torch.float32 else 8)
+    W, idx, p, _ = eb_inputs(B, L, 500, D, dtype, seed=B + L, with_grad=False)
+    idx = idx.clamp_min(1)
+    expect = ref.eb_forward(idx, W, p)
+    if L > 2:
+        p0 = p.clone()
+        p0[:, 1] = 0
+        expect = ref.eb_forward(idx, W, p0)
+        idx[:, 1] = torch.where(torch.arange(B) % 2 == 0, -1, 500)
+        p[:, 1] = float("nan")
+    W[0] = float("inf")
+    out = eb.eb_forward(*_dev(idx, W, p, device=device))
+    cond = ref.eb_forward(idx.clamp(1, 499), W.abs(), p.abs().nan_to_num(0.0))
+    assert_rel_close(out, expect, REL_TOL[dtype], f"forward {dtype} {B,L,D}", cond=cond)
+
+
 def test_forward_empty(device):
     from modelos_amd import embedding_bag as eb
 
