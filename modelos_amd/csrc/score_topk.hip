@@ -579,8 +579,8 @@ __device__ __forceinline__ void cartesian_rows(const typename Sel<TIN>::Key* l0r
 // ---------------------------------------------------------------------------
 template <typename TIN, int IDW, int TM, int KSC>
 __global__ __launch_bounds__(kThreads) void pkm_score_topk_kernel(
-    const TIN* __restrict__ Q, const TIN* __restrict__ Kt, int kpack, int64_t Ntok, int H, int n, int half, int knn,
-    TIN* __restrict__ out_scores, int64_t* __restrict__ out_idx, int64_t* __restrict__ out_i1,
+    const TIN* __restrict__ Q, const TIN* __restrict__ Kt, int kpack, int hsplit, int64_t Ntok, int H, int n, int half,
+    int knn, TIN* __restrict__ out_scores, int64_t* __restrict__ out_idx, int64_t* __restrict__ out_i1,
     int64_t* __restrict__ out_i2, TIN* __restrict__ out_s1, TIN* __restrict__ out_s2) {
   typedef Sel<TIN> SL;
   typedef typename SL::Store Store;
@@ -603,8 +603,11 @@ __global__ __launch_bounds__(kThreads) void pkm_score_topk_kernel(
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int h = (int)(blockIdx.x % (unsigned)H);
-  const int64_t t0 = (int64_t)(blockIdx.x / (unsigned)H) * TM;
+  // hsplit (32-bit keys only): a workgroup takes one half, halves outermost of a tile's 2 H workgroups
+  const unsigned HG = hsplit ? 2u * (unsigned)H : (unsigned)H;
+  const int h = (int)(blockIdx.x % HG % (unsigned)H);
+  const int hc0 = hsplit ? (int)(blockIdx.x % HG / (unsigned)H) : 0, hc1 = hsplit ? hc0 + 1 : 2;
+  const int64_t t0 = (int64_t)(blockIdx.x / HG) * TM;
   const ScoreLds L = score_lds_layout(TM, n, half, knn, (int)sizeof(Store), (int)sizeof(Key));
   const TileMap M = tile_map(n);
   Store* S = (Store*)smem;
@@ -652,7 +655,7 @@ __global__ __launch_bounds__(kThreads) void pkm_score_topk_kernel(
   const int cx = (LPR == 8 && NCH % (2 * LPR) == 0) ? (r & 1) : 0;
 
 #pragma unroll 1
-  for (int hc = 0; hc < 2; ++hc) {
+  for (int hc = hc0; hc < hc1; ++hc) {
     const TIN* Kc = Kt + (int64_t)(2 * h + hc) * n * half;
     // ---- A0: stage the query half [TM][half] (zeros past the last token)
     if constexpr (KSC > 0 && (TM * 4 * KSC) % kThreads == 0) {
@@ -911,8 +914,9 @@ __global__ __launch_bounds__(kThreads) void pkm_score_topk_kernel(
     }
     const uint32_t incl = group_scan<LPR>(cnt, sub);
     const uint32_t total = group_sum<LPR>(cnt);
-    const bool overflow = total > (uint32_t)L.cap;
-    if (!overflow) {
+    // (the zero scores of rows past the last token all tie: no exact search for them)
+    const bool overflow = live && total > (uint32_t)L.cap;
+    if (live && !overflow) {
       uint32_t p = incl - cnt;
       // column of element j of chunk c: c * (E / slots) + off[j] when a chunk
       // of E elements spans whole groups of slots positions
@@ -943,7 +947,7 @@ __global__ __launch_bounds__(kThreads) void pkm_score_topk_kernel(
     }
     __builtin_amdgcn_wave_barrier();
     auto to_list = [&](uint32_t rank, Key k) { list[rank] = k; };
-    if (!overflow) {
+    if (live && !overflow) {
       if (L.cap <= 8 * LPR)
         group_rank<Key, LPR, 8>(cand, total, knn, sub, to_list);
       else
@@ -972,7 +976,10 @@ __global__ __launch_bounds__(kThreads) void pkm_score_topk_kernel(
       if (live) {
         for (int j = sub; j < knn; j += LPR) {
           const Key k = list[j];
-          out_idx[orow + j] = (int64_t)k;
+          if constexpr (kSplitC)
+            ((uint32_t*)(out_idx + orow + j))[0] = (uint32_t)k;
+          else
+            out_idx[orow + j] = (int64_t)k;
           if (out_i1 != nullptr) out_i1[orow + j] = (int64_t)SL::key_idx(k);
         }
       }
@@ -1084,7 +1091,8 @@ __global__ __launch_bounds__(kThreads) void pkm_score_cartesian_kernel(int64_t r
 }
 
 // ---------------------------------------------------------------------------
-// Streaming scoring: bfloat16 dot scores, knn <= 32, half key dim 128 or 256.
+// Streaming scoring: bfloat16 dot scores, knn <= 32, half key dim 128 or 256,
+// more tokens than few_tokens_tile leaves to the tile kernel.
 //
 // One workgroup of 8 waves, two per SIMD, owns 256 tokens of one (head, half):
 // while one wave of a SIMD runs its selection on the vector ALUs, the other
@@ -1583,10 +1591,14 @@ __host__ inline size_t lds_bytes(int half) {
 
 }  // namespace stream
 
-constexpr int kCartLpr = 8;  // lanes per row of the cartesian kernel
-__host__ inline size_t cartesian_lds_bytes(int knn) {
+// Lanes per row of the cartesian kernel: 8 in bulk; 32 up to 8192 rows, where
+// the row's serial chain is what it takes (knn 32, up to 4096 rows: scoring +
+// cartesian 2 to 4 us less; knn 64, 4096 rows 75 -> 63 us, 8192 rows 102 ->
+// 95; 16384 rows of knn 32 72 -> 80).
+constexpr int64_t kCartWideRows = 8192;
+__host__ inline size_t cartesian_lds_bytes(int knn, int lpr) {
   const int kl = (knn + 3) & ~3;
-  return (size_t)(kThreads / kCartLpr) * (size_t)(3 * kl + score_cap(knn, kCartLpr) + 4) * 4;
+  return (size_t)(kThreads / lpr) * (size_t)(3 * kl + score_cap(knn, lpr) + 4) * 4;
 }
 
 // Dynamic LDS above 64 KiB is enabled once per device and kernel (idempotent,
@@ -1608,37 +1620,43 @@ static int enable_lds(const void* fn, int bytes, std::atomic<uint64_t>& done, co
 // The cartesian step of the packed lists (32-bit keys: bf16 scores). The LDS
 // attribute is set once per device, to the device maximum, so that every
 // knn's layout fits.
-template <typename TIN>
-static int launch_cartesian(int64_t Ntok, int H, int n, int knn, int lds_max, void* out_scores, int64_t* out_idx,
-                            hipStream_t st) {
+template <typename TIN, int LPR>
+static int launch_cartesian_lpr(int64_t rows, int n, int knn, int lds_max, void* out_scores, int64_t* out_idx,
+                                hipStream_t st) {
   static_assert(sizeof(typename Sel<TIN>::Key) == 4, "packed lists need 32-bit keys");
   static std::atomic<uint64_t> cart_lds_enabled{0};
-  const size_t cl = cartesian_lds_bytes(knn);
+  const size_t cl = cartesian_lds_bytes(knn, LPR);
   if ((int)cl > lds_max)
     return pkm_set_error(PKM_ERR_UNSUPPORTED, "pkm_score_topk: knn %d needs %zu bytes of LDS for the cartesian step",
                          knn, cl);
-  const int rc = enable_lds((const void*)pkm_score_cartesian_kernel<TIN, kCartLpr>, lds_max, cart_lds_enabled,
+  const int rc = enable_lds((const void*)pkm_score_cartesian_kernel<TIN, LPR>, lds_max, cart_lds_enabled,
                             "pkm_score_topk");
   if (rc != PKM_OK) return rc;
-  const int64_t rows = Ntok * H;
-  const int64_t cblocks = (rows + kThreads / kCartLpr - 1) / (kThreads / kCartLpr);
-  hipLaunchKernelGGL((pkm_score_cartesian_kernel<TIN, kCartLpr>), dim3((unsigned)cblocks), dim3(kThreads), cl, st,
-                     rows, n, knn, (TIN*)out_scores, out_idx);
+  const int64_t cblocks = (rows + kThreads / LPR - 1) / (kThreads / LPR);
+  hipLaunchKernelGGL((pkm_score_cartesian_kernel<TIN, LPR>), dim3((unsigned)cblocks), dim3(kThreads), cl, st, rows, n,
+                     knn, (TIN*)out_scores, out_idx);
   return PKM_OK;
+}
+template <typename TIN>
+static int launch_cartesian(int64_t Ntok, int H, int n, int knn, int lds_max, void* out_scores, int64_t* out_idx,
+                            hipStream_t st) {
+  const int64_t rows = Ntok * H;
+  return rows <= kCartWideRows ? launch_cartesian_lpr<TIN, 32>(rows, n, knn, lds_max, out_scores, out_idx, st)
+                               : launch_cartesian_lpr<TIN, 8>(rows, n, knn, lds_max, out_scores, out_idx, st);
 }
 
 template <typename TIN, int IDW, int TM, int KSC>
-static int launch_score_tm(const void* q, const void* keys, int kpack, int64_t Ntok, int H, int n, int half, int knn,
+static int launch_score_tm(const void* q, const void* keys, int kpack, int hsplit, int64_t Ntok, int H, int n, int half, int knn,
                            size_t lds, int lds_max, void* out_scores, int64_t* out_idx, int64_t* out_i1,
                            int64_t* out_i2, void* out_s1, void* out_s2, hipStream_t st) {
   static std::atomic<uint64_t> lds_enabled{0};
   int rc = enable_lds((const void*)pkm_score_topk_kernel<TIN, IDW, TM, KSC>, lds_max, lds_enabled, "pkm_score_topk");
   if (rc != PKM_OK) return rc;
-  const int64_t blocks = ((Ntok + TM - 1) / TM) * H;
+  const int64_t blocks = ((Ntok + TM - 1) / TM) * H * (hsplit ? 2 : 1);
   {
     KernelSpan span("score_topk", st);
     hipLaunchKernelGGL((pkm_score_topk_kernel<TIN, IDW, TM, KSC>), dim3((unsigned)blocks), dim3(kThreads), lds, st,
-                       (const TIN*)q, (const TIN*)keys, kpack, Ntok, H, n, half, knn, (TIN*)out_scores, out_idx, out_i1,
+                       (const TIN*)q, (const TIN*)keys, kpack, hsplit, Ntok, H, n, half, knn, (TIN*)out_scores, out_idx, out_i1,
                        out_i2, (TIN*)out_s1, (TIN*)out_s2);
   }
   if constexpr (sizeof(typename Sel<TIN>::Key) == 4) return launch_cartesian<TIN>(Ntok, H, n, knn, lds_max, out_scores, out_idx, st);
@@ -1666,38 +1684,38 @@ static int launch_stream(const void* q, const void* keys, int64_t Ntok, int H, i
 // Kernel variant for (TM, k-steps per half): the k-step counts of the common
 // half key dims (128, 256, 512 elements) are compile-time.
 template <typename TIN, int IDW, int TM>
-static int launch_score_ks(const void* q, const void* keys, int kpack, int64_t Ntok, int H, int n, int half, int knn,
+static int launch_score_ks(const void* q, const void* keys, int kpack, int hsplit, int64_t Ntok, int H, int n, int half, int knn,
                            size_t lds, int lds_max, void* out_scores, int64_t* out_idx, int64_t* out_i1,
                            int64_t* out_i2, void* out_s1, void* out_s2, hipStream_t st) {
   switch (half / Sel<TIN>::KSTEP) {
     case 4:
-      return launch_score_tm<TIN, IDW, TM, 4>(q, keys, kpack, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx,
+      return launch_score_tm<TIN, IDW, TM, 4>(q, keys, kpack, hsplit, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx,
                                               out_i1, out_i2, out_s1, out_s2, st);
     case 8:
-      return launch_score_tm<TIN, IDW, TM, 8>(q, keys, kpack, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx,
+      return launch_score_tm<TIN, IDW, TM, 8>(q, keys, kpack, hsplit, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx,
                                               out_i1, out_i2, out_s1, out_s2, st);
     case 16:
-      return launch_score_tm<TIN, IDW, TM, 16>(q, keys, kpack, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx,
+      return launch_score_tm<TIN, IDW, TM, 16>(q, keys, kpack, hsplit, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx,
                                                out_i1, out_i2, out_s1, out_s2, st);
     default:
-      return launch_score_tm<TIN, IDW, TM, 0>(q, keys, kpack, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx,
+      return launch_score_tm<TIN, IDW, TM, 0>(q, keys, kpack, hsplit, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx,
                                               out_i1, out_i2, out_s1, out_s2, st);
   }
 }
 
 template <typename TIN, int IDW>
-static int launch_score(int TM, const void* q, const void* keys, int kpack, int64_t Ntok, int H, int n, int half, int knn,
+static int launch_score(int TM, const void* q, const void* keys, int kpack, int hsplit, int64_t Ntok, int H, int n, int half, int knn,
                         size_t lds, int lds_max, void* out_scores, int64_t* out_idx, int64_t* out_i1,
                         int64_t* out_i2, void* out_s1, void* out_s2, hipStream_t st) {
   switch (TM) {
     case 64:
-      return launch_score_ks<TIN, IDW, 64>(q, keys, kpack, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx, out_i1,
+      return launch_score_ks<TIN, IDW, 64>(q, keys, kpack, hsplit, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx, out_i1,
                                            out_i2, out_s1, out_s2, st);
     case 32:
-      return launch_score_ks<TIN, IDW, 32>(q, keys, kpack, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx, out_i1,
+      return launch_score_ks<TIN, IDW, 32>(q, keys, kpack, hsplit, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx, out_i1,
                                            out_i2, out_s1, out_s2, st);
     default:
-      return launch_score_ks<TIN, IDW, 16>(q, keys, kpack, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx, out_i1,
+      return launch_score_ks<TIN, IDW, 16>(q, keys, kpack, hsplit, Ntok, H, n, half, knn, lds, lds_max, out_scores, out_idx, out_i1,
                                            out_i2, out_s1, out_s2, st);
   }
 }
@@ -1725,6 +1743,29 @@ __global__ __launch_bounds__(256) void score_keys_pack_kernel(const uint4* __res
   const int64_t tile = o / tsz;
   const int w = (int)(o - tile * tsz);
   P[o] = K[tile * tsz + (int64_t)(w & 15) * CH + (w >> 4)];
+}
+}  // namespace pkm
+
+namespace pkm {
+// Tokens per tile of the tile kernel where the tokens are too few to fill the
+// chip: the smallest tile whose workgroups fit it in one round (bf16: one half
+// each), 0 where not even the largest tile's do. The scores are the same bits
+// as the streaming kernel's (both sum a dot product in ascending k-steps of
+// the matrix cores), which takes a whole workgroup and the same time for 1 to
+// 256 tokens of a (head, half). Scoring + cartesian step, bf16, knn 32, half
+// 256, streaming -> this rule's tile: 8 heads x 1024 keys, 8 tokens 90 -> 33
+// us, 512 tokens 68 -> 43, 1024 tokens 70 -> 49 (2048: 73 against 74, past
+// the rule); 4 heads x 512 keys, 256 tokens 49 -> 30, 2048 tokens 51 -> 40 (4096: 54
+// against 64). The selection's threshold needs groups enough for knn of their
+// maxima to be a tight bound: with fewer than 2 knn groups most rows take the
+// exact search and the streaming kernel is the faster one (256 keys, knn 32,
+// 512 tokens: 38 against 47).
+static int few_tokens_tile(int64_t tokens, int H, int n, int knn, int dtype, int max_tile) {
+  if (dtype == PKM_DTYPE_BF16 && n < 16 * knn) return 0;
+  const int64_t per_tile = dtype == PKM_DTYPE_BF16 ? 2 * (int64_t)H : H;
+  for (int tile = 16; tile <= max_tile; tile *= 2)
+    if ((tokens + tile - 1) / tile * per_tile <= 256) return tile;
+  return 0;
 }
 }  // namespace pkm
 
@@ -1767,8 +1808,13 @@ static int score_topk_impl(const void* query, const void* keys, int64_t num_toke
     if (rc != PKM_OK) return rc;
     return pkm_check_launch("pkm_score_topk");
   }
-  if (dtype == PKM_DTYPE_BF16 && score_type == PKM_SCORE_DOT && knn <= stream::kNet && (half == 128 || half == 256) &&
-      (int)stream::lds_bytes((int)half) <= lds_max) {
+  const int H = (int)heads, n = (int)n_keys, hf = (int)half, k = (int)knn;
+  int TM = 64;
+  while (TM > 16 && (score_lds_layout(TM, n, hf, k, esz, key_bytes).total > lds_max || n > score_max_n(TM, esz)))
+    TM /= 2;
+  const int few = few_tokens_tile(num_tokens, H, n, k, dtype, TM);
+  if (!few && dtype == PKM_DTYPE_BF16 && score_type == PKM_SCORE_DOT && knn <= stream::kNet &&
+      (half == 128 || half == 256) && (int)stream::lds_bytes((int)half) <= lds_max) {
     const int64_t blocks = ((num_tokens + stream::kTok - 1) / stream::kTok) * 2 * heads;
     PKM_REQUIRE(blocks < ((int64_t)1 << 31), PKM_ERR_INVALID_ARGUMENT, "pkm_score_topk: grid too large");
     const bool sub = out_sub_scores1 != nullptr || out_sub_scores2 != nullptr;
@@ -1779,11 +1825,9 @@ static int score_topk_impl(const void* query, const void* keys, int64_t num_toke
     if (rc != PKM_OK) return rc;
     return pkm_check_launch("pkm_score_topk");
   }
-  int TM = 64;
-  while (TM > 16 && (score_lds_layout(TM, (int)n_keys, (int)half, (int)knn, esz, key_bytes).total > lds_max ||
-                     n_keys > score_max_n(TM, esz)))
-    TM /= 2;
-  const int lds = score_lds_layout(TM, (int)n_keys, (int)half, (int)knn, esz, key_bytes).total;
+  if (few) TM = few;
+  const int hsplit = few != 0 && dtype == PKM_DTYPE_BF16;
+  const int lds = score_lds_layout(TM, n, hf, k, esz, key_bytes).total;
   if (lds > lds_max) {  // a tile too large for the device's LDS: the generic kernel
     const int rc = score_topk_generic(query, keys, num_tokens, heads, n_keys, half, knn, score_type, dtype, out_scores,
                                       out_indices, out_sub_indices1, out_sub_indices2, out_sub_scores1,
@@ -1794,7 +1838,6 @@ static int score_topk_impl(const void* query, const void* keys, int64_t num_toke
   const int64_t blocks = ((num_tokens + TM - 1) / TM) * heads;
   PKM_REQUIRE(blocks < ((int64_t)1 << 31), PKM_ERR_INVALID_ARGUMENT, "pkm_score_topk: grid too large");
   int rc;
-  const int H = (int)heads, n = (int)n_keys, hf = (int)half, k = (int)knn;
   // with a workspace of the keys' size: the keys packed tile-major first (one
   // pass over the table), so the kernel's key loads use whole cache lines
   const size_t key_bytes_all = (size_t)(2 * heads * n_keys) * (size_t)half * (dtype == PKM_DTYPE_BF16 ? 2 : 4);
@@ -1808,18 +1851,18 @@ static int score_topk_impl(const void* query, const void* keys, int64_t num_toke
   }
   if (dtype == PKM_DTYPE_BF16) {
     rc = score_type == PKM_SCORE_DOT
-             ? launch_score<bf16_t, 0>(TM, query, keys, kpack, num_tokens, H, n, hf, k, (size_t)lds, lds_max, out_scores,
+             ? launch_score<bf16_t, 0>(TM, query, keys, kpack, hsplit, num_tokens, H, n, hf, k, (size_t)lds, lds_max, out_scores,
                                        out_indices, out_sub_indices1, out_sub_indices2, out_sub_scores1,
                                        out_sub_scores2, st)
-             : launch_score<bf16_t, 1>(TM, query, keys, kpack, num_tokens, H, n, hf, k, (size_t)lds, lds_max, out_scores,
+             : launch_score<bf16_t, 1>(TM, query, keys, kpack, hsplit, num_tokens, H, n, hf, k, (size_t)lds, lds_max, out_scores,
                                        out_indices, out_sub_indices1, out_sub_indices2, out_sub_scores1,
                                        out_sub_scores2, st);
   } else {
     rc = score_type == PKM_SCORE_DOT
-             ? launch_score<float, 0>(TM, query, keys, kpack, num_tokens, H, n, hf, k, (size_t)lds, lds_max, out_scores,
+             ? launch_score<float, 0>(TM, query, keys, kpack, hsplit, num_tokens, H, n, hf, k, (size_t)lds, lds_max, out_scores,
                                       out_indices, out_sub_indices1, out_sub_indices2, out_sub_scores1,
                                       out_sub_scores2, st)
-             : launch_score<float, 1>(TM, query, keys, kpack, num_tokens, H, n, hf, k, (size_t)lds, lds_max, out_scores,
+             : launch_score<float, 1>(TM, query, keys, kpack, hsplit, num_tokens, H, n, hf, k, (size_t)lds, lds_max, out_scores,
                                       out_indices, out_sub_indices1, out_sub_indices2, out_sub_scores1,
                                       out_sub_scores2, st);
   }

@@ -169,3 +169,56 @@ def test_single_sub_score_output_through_c_abi(device, which, dtype):
     torch.cuda.synchronize()
     assert torch.equal(idx, full[1]) and torch.equal(scores, full[0])
     assert torch.equal(s_out, full[4] if which == 1 else full[5])
+
+
+def _repeat_tokens(q, tokens):
+    return q.repeat((tokens + q.shape[0] - 1) // q.shape[0], 1, 1)[:tokens].contiguous()
+
+
+# Few tokens run on the tile kernel (the smallest tile whose workgroups fit the
+# chip in one round), many on the streaming one: each token's outputs are the
+# same bits on both, for the streaming kernel's own cases too (the others of
+# this file have few tokens). 4100 and 4353 tokens of 2 heads are past the
+# tile kernel's rule, 1, 16, 17, 1025 and 2049 take its 16-, 32- and 64-token tiles.
+@pytest.mark.parametrize("knn", [1, 7, 16, 31, 32])
+@pytest.mark.parametrize("case", ["random", "zero", "increasing", "decreasing", "increasing_negative", "signed_zero"])
+def test_few_and_many_tokens_agree(device, case, knn):
+    H, n, half = 2, 1024 if case in ("increasing", "decreasing") else 512, 128 if case == "signed_zero" else 256
+    N = 97
+    v = (torch.arange(n, dtype=torch.float32) + 1) / 16
+    g = gen(200 + knn)
+    if case in ("random", "zero"):
+        q = torch.randn((N, H, 2 * half), generator=g).to(torch.bfloat16)
+        k = (torch.randn((2 * H * n, half), generator=g) * half**-0.5).to(torch.bfloat16)
+        if case == "zero":
+            q.zero_()
+    else:
+        vals = {"increasing": v, "decreasing": v.flip(0), "increasing_negative": -v.flip(0)}.get(case)
+        if vals is None:
+            vals = torch.zeros(n)
+            vals[1::2] = -0.0
+            vals[::97] = 1.0
+        q, k = _one_hot_keys(N, H, n, half, vals, seed=201)
+    many = _run(_repeat_tokens(q, 4353), k, H, knn, device)
+    for tokens in (1, 16, 17, 1025, 2049, 4100):
+        few = _run(_repeat_tokens(q, tokens), k, H, knn, device)
+        for a, b in zip(few, many):
+            assert torch.equal(a, b[: a.shape[0]]), f"{case} knn {knn} tokens {tokens}"
+
+
+# The rule's other routes: more lanes per row in the cartesian step up to 8192
+# rows, smaller tiles of float32 and of key dims the streaming kernel does not
+# take, dead rows of a tile (their equal scores select nothing).
+@pytest.mark.parametrize("dtype,score,half,knn", [(torch.float32, "idw", 128, 16), (torch.float32, "dot", 64, 33),
+                                                  (torch.bfloat16, "dot", 64, 24), (torch.bfloat16, "idw", 128, 32),
+                                                  (torch.bfloat16, "dot", 256, 64)], ids=str)
+def test_few_token_tiles_agree(device, dtype, score, half, knn):
+    H, n, N = 3, 1024, 6001
+    g = gen(300 + knn)
+    q = (torch.randn((N, H, 2 * half), generator=g) * half**-0.5).to(dtype)
+    k = (torch.randn((2 * H * n, half), generator=g) * half**-0.5).to(dtype)
+    many = score_topk(q.to(device), k.to(device), H, knn, score, sub_outputs=True)
+    for tokens in (1, 5, 33, 700, 1400, 2700):
+        few = score_topk(q[:tokens].to(device), k.to(device), H, knn, score, sub_outputs=True)
+        for a, b in zip(few, many):
+            assert torch.equal(a, b[: a.shape[0]]), f"tokens {tokens}"
