@@ -21,7 +21,7 @@ def _require_device(*tensors: Optional[torch.Tensor]) -> torch.device:
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 f"PKM HIP kernels need ROCm device tensors, got a tensor on {t.device} "
                 "(this implementation has no CPU path)"
