@@ -50,7 +50,8 @@ const char* pkm_last_error_string(void);
 /*
  * Weighted embedding bag, forward (mode "sum").
  *   out[b, :] = sum_{j < bag_size} psw[b, j] * weight[indices[b, j], :]
- * Accumulates in float32 in j order and rounds once to weight's dtype.
+ * Accumulates in float32 in j order (for bags too few to fill the GPU in up to
+ * 16 partial sums, added in a fixed order) and rounds once to weight's dtype.
  * psw may be NULL (psw_dtype PKM_DTYPE_NONE): all weights are 1.
  * out: [bags, dim] in weight_dtype.
  *
@@ -506,6 +507,19 @@ int pkm_swilu_fwd(const void* e, const void* s, int64_t n, int dtype, void* h, v
  */
 int pkm_swilu_bwd(const void* dh, const void* e, const void* s, int64_t n, int dtype, void* de, void* ds,
                   void* stream);
+
+/*
+ * A Linear over a few rows: y[i, o] = bf16(sum_k x[i, k] * weight[o, k] + bias[o]),
+ * float32 sums, one rounding. x [rows, in_features], weight [out_features,
+ * in_features], bias [out_features] or NULL, y [rows, out_features]; bfloat16,
+ * rows <= 64, in_features a multiple of 32, out_features of 16, x and weight
+ * 16-byte aligned: PKM_ERR_UNSUPPORTED otherwise.
+ *
+ * Replaces F.linear of the value projections (pkm/memory.py:222-229) for the
+ * few rows of a decode step.
+ */
+int pkm_linear_rows(const void* x, const void* weight, const void* bias, int64_t rows, int64_t in_features,
+                    int64_t out_features, int dtype, void* y, void* stream);
 
 /* Workspace bytes pkm_rmsnorm_bwd needs for these sizes. */
 size_t pkm_rmsnorm_bwd_workspace_size(int64_t rows, int64_t dim);

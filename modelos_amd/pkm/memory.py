@@ -61,7 +61,7 @@ class _Linear(torch.autograd.Function):
     fp32 gradients), as nn.Linear's autograd does."""
 
     @staticmethod
-    def forward(ctx, x, weight, bias):
+    def forward(ctx, x, weight, bias, few_rows):
         ctx.dtypes = (x.dtype, weight.dtype, bias.dtype if bias is not None else None)
         dev = x.device.type
         autocast = torch.is_autocast_enabled(dev)
@@ -71,6 +71,11 @@ class _Linear(torch.autograd.Function):
             bias = bias.to(dt) if bias is not None else None
         ctx.save_for_backward(x, weight)
         ctx.has_bias = bias is not None
+        if few_rows and _rows_kernel_takes(x, weight, bias):
+            y = torch.empty((x.shape[0], weight.shape[0]), dtype=x.dtype, device=x.device)
+            _lib.call("pkm_linear_rows", _lib.ptr(x), _lib.ptr(weight), _lib.ptr(bias), x.shape[0], x.shape[1],
+                      weight.shape[0], _lib.dtype_code(x), _lib.ptr(y), _lib.stream_of(x.device))
+            return y
         if not autocast:  # (entering and leaving the context costs 5 us a call)
             return F.linear(x, weight, bias)
         with torch.autocast(dev, enabled=False):
@@ -98,7 +103,7 @@ class _Linear(torch.autograd.Function):
             gw = gw.to(w_dt)
         if ctx.has_bias and ctx.needs_input_grad[2]:
             gb = _column_sum(g).to(b_dt)
-        return gx, gw, gb
+        return gx, gw, gb, None
 
 
 def _column_sum(g: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.Tensor:
@@ -123,9 +128,31 @@ def _column_sum(g: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.
     return out
 
 
-def _linear(layer: nn.Linear, x: torch.Tensor) -> torch.Tensor:
-    """layer(x) for a 2-D x, through _Linear."""
-    return _Linear.apply(x, layer.weight, layer.bias)
+_PLAIN_TENSORS = (torch.Tensor, nn.Parameter)
+
+
+def _rows_kernel_takes(x, weight, bias) -> bool:
+    """Whether pkm_linear_rows serves these operands: up to 64 bf16 rows of
+    plain, contiguous, aligned tensors on one GPU (above, the BLAS's tiles
+    are full: 64 rows of 1024 x 1024 take 5 us here and 7 us there)."""
+    if x.dim() != 2 or not 0 < x.shape[0] <= 64 or x.dtype != torch.bfloat16 or not x.is_cuda:
+        return False
+    if type(x) not in _PLAIN_TENSORS or type(weight) not in _PLAIN_TENSORS or x.shape[1] != weight.shape[1]:
+        return False
+    if bias is not None and (type(bias) not in _PLAIN_TENSORS or bias.dtype != x.dtype or bias.device != x.device
+                             or not bias.is_contiguous()):
+        return False
+    return (weight.dtype == x.dtype and weight.device == x.device and x.is_contiguous() and weight.is_contiguous()
+            and x.shape[1] % 32 == 0 and weight.shape[0] % 16 == 0 and x.data_ptr() % 16 == 0
+            and weight.data_ptr() % 16 == 0)
+
+
+def _linear(layer: nn.Linear, x: torch.Tensor, few_rows: bool = False) -> torch.Tensor:
+    """layer(x) for a 2-D x, through _Linear. few_rows: small inputs may take
+    pkm_linear_rows, whose sums have another order than the BLAS's. The query
+    projection does not: one query element rounded the other way reorders
+    the selection behind it."""
+    return _Linear.apply(x, layer.weight, layer.bias, few_rows)
 
 logger = getLogger()
 
@@ -294,9 +321,10 @@ class HashingMemory(nn.Module):
         if not self.use_peer_variant:
             output = self.values(indices, scores)  # [bs, v_dim]
             if self.v_proj and not self.swilu_proj:
-                output = _linear(self.value_proj, output)
+                output = _linear(self.value_proj, output, True)
             if self.swilu_proj:
-                output = _linear(self.value_proj, swilu_gate(output, _linear(self.swilu_projection, input)))
+                gate = _linear(self.swilu_projection, input, True)
+                output = _linear(self.value_proj, swilu_gate(output, gate), True)
         else:
             # PEER variant (memory.py:231-237): per-slot expert vectors
             u = self.values_u(indices)  # [bs, heads * knn, v_dim]

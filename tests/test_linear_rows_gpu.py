@@ -1,0 +1,55 @@
+"""pkm_linear_rows (a Linear over a few bf16 rows) against float64.
+
+The value Linears of a decode step: row counts around the 16-row tiles, input
+widths of fewer k-steps than waves, of a ragged share per wave and of many, one
+tile of outputs and several, with and without a bias. Bound: one bf16 rounding
+(2^-9 relative, 2^-8 with the bias of another magnitude) of float32 sums whose
+error is far below it, taken relative to the sum of |terms|.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from modelos_amd import _lib
+from modelos_amd.pkm import memory
+from tests.helpers import gen
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("rows,fin,fout", [(1, 32, 16), (8, 1024, 1024), (15, 96, 48), (16, 288, 16), (17, 512, 1024),
+                                           (33, 1056, 32), (64, 4096, 64)])
+def test_against_float64(device, rows, fin, fout, bias):
+    g = gen(rows + fin)
+    lin = torch.nn.Linear(fin, fout, bias=bias)
+    with torch.no_grad():
+        lin.weight.copy_(torch.randn((fout, fin), generator=g) * fin**-0.5)
+        if bias:
+            lin.bias.copy_(torch.randn(fout, generator=g))
+    lin = lin.to(device=device, dtype=torch.bfloat16)
+    x = torch.randn((rows, fin), generator=g).to(torch.bfloat16).to(device)
+    assert memory._rows_kernel_takes(x, lin.weight, lin.bias)
+    y = memory._linear(lin, x, True)
+    w64, x64 = lin.weight.detach().double(), x.double()
+    b64 = lin.bias.detach().double() if bias else torch.zeros(fout, dtype=torch.float64, device=device)
+    expect = x64 @ w64.t() + b64
+    bound = (x64.abs() @ w64.abs().t() + b64.abs()) * 2.0**-20 + expect.abs() * 2.0**-8
+    assert ((y.double() - expect).abs() <= bound).all()
+    assert torch.equal(y, memory._linear(lin, x, True))
+
+
+def test_what_it_does_not_take(device):
+    lin = torch.nn.Linear(64, 32).to(device=device, dtype=torch.bfloat16)
+    x = torch.randn((65, 64), device=device).to(torch.bfloat16)
+    assert not memory._rows_kernel_takes(x, lin.weight, lin.bias)  # rows
+    assert memory._rows_kernel_takes(x[:64], lin.weight, lin.bias)
+    assert not memory._rows_kernel_takes(x[:8, ::2], lin.weight[:, :32], lin.bias)  # strides
+    assert not memory._rows_kernel_takes(x[:8].float(), lin.weight.float(), lin.bias.float())
+    assert not memory._rows_kernel_takes(x.reshape(-1)[1:8 * 64 + 1].view(8, 64), lin.weight, lin.bias)  # alignment
+    y = torch.empty((8, 32), dtype=torch.bfloat16, device=device)
+    for rows, fin, fout, code in ((65, 64, 32, 1), (8, 48, 32, 1), (8, 64, 24, 1), (8, 64, 32, 0)):
+        with pytest.raises(_lib.PkmError):
+            _lib.call("pkm_linear_rows", _lib.ptr(x), _lib.ptr(lin.weight), None, rows, fin, fout, code, _lib.ptr(y),
+                      _lib.stream_of(x.device))
