@@ -28,9 +28,9 @@ def _ref(x):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16], ids=["bf16", "f32", "f16"])
 @pytest.mark.parametrize("shape", [(131072, 32), (300, 64), (77, 7), (5, 1), (3, 4, 33), (101, 8), (99, 16), (50, 4),
-                                   (8192, 64 * 4), (33, 65), (7, 1000), (3, 5000), (31, 128), (13, 512), (2, 24)],
+                                   (8192, 64 * 4), (33, 65), (7, 1000), (3, 5000), (31, 128), (13, 512)],
                          ids=["layer", "k64", "k7", "k1", "3d-k33", "k8", "k16", "k4", "fw-h4k64", "k65", "k1000",
-                              "k5000", "k128", "k512", "k24"])
+                              "k5000", "k128", "k512"])
 def test_matches_torch(device, dtype, shape):
     g = gen(11)
     x = (torch.randn(shape, generator=g) * 4).to(dtype).to(device)
