@@ -44,11 +44,9 @@
 #include <mutex>
 #include <type_traits>
 
-#include "pkm_common.h"
+#include "eb_reduce.h"
 
 namespace pkm {
-
-constexpr int kHeavyT = 256;  // chunk length and light/heavy row threshold
 
 // ---------------------------------------------------------------------------
 // The fast-weight SGD step in the reduction's epilogue (pkm_eb_bwd_sgd): a
@@ -207,6 +205,56 @@ __global__ __launch_bounds__(256) void scan_reduce_kernel(const uint32_t* __rest
   if (threadIdx.x == 0) parts[blockIdx.x] = tot;
 }
 
+// One block: in-place exclusive prefix sum of data[0..n), data[n] <- the total,
+// 8192 words a step, the next step's loaded while this one's are summed.
+constexpr int64_t kScanOneMax = 16384;  // (two steps: 9.8 us)
+__global__ __launch_bounds__(1024) void scan_one_kernel(uint32_t* __restrict__ data, int n) {
+  __shared__ uint32_t wtot[2][16];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint32_t carry = 0;
+  uint32_t next[8];
+  auto load = [&](int base) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int p = base + (int)threadIdx.x * 8 + i;
+      next[i] = p < n ? data[p] : 0u;
+    }
+  };
+  load(0);
+#pragma unroll 1
+  for (int base = 0, k = 0; base < n; base += 8192, k ^= 1) {
+    uint32_t v[8], s = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[i] = next[i];
+      s += v[i];
+    }
+    load(base + 8192);
+    uint32_t x = s;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = (uint32_t)__shfl_up((int)x, o);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) wtot[k][w] = x;
+    __syncthreads();  // (two buffers: the next step's totals don't meet this one's readers)
+    uint32_t run = carry + x - s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t t = wtot[k][i];
+      run += i < w ? t : 0u;
+      carry += t;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int p = base + (int)threadIdx.x * 8 + i;
+      if (p < n) data[p] = run;
+      run += v[i];
+    }
+  }
+  if (threadIdx.x == 0) data[n] = carry;
+}
+
 // Single block: exclusive prefix sum of the per-tile sums, in place.
 __global__ __launch_bounds__(256) void scan_parts_kernel(uint32_t* __restrict__ parts, int64_t nparts) {
   __shared__ uint32_t lds4[4];
@@ -290,9 +338,10 @@ __global__ __launch_bounds__(256) void radix_hist_kernel(const int64_t* __restri
                                                          const uint32_t* __restrict__ keys, int64_t N,
                                                          const uint32_t* __restrict__ nvalid, int64_t K, int shift,
                                                          uint32_t* __restrict__ hist, int64_t ntiles,
-                                                         uint32_t* __restrict__ invalid) {
+                                                         uint32_t* __restrict__ invalid, FillShare fill = FillShare{}) {
   constexpr int R = 1 << BITS;
   __shared__ uint32_t h[R];
+  if (fill_share(fill)) return;
   for (int d = threadIdx.x; d < R; d += 256) h[d] = 0;
   __syncthreads();
   const uint32_t nv = FIRST ? 0u : *nvalid;
@@ -345,7 +394,8 @@ __global__ __launch_bounds__(256) void radix_scatter_kernel(const int64_t* __res
                                                             uint32_t* __restrict__ vals_out, SegTab seg = SegTab{},
                                                             uint2* __restrict__ meta = nullptr,
                                                             const void* __restrict__ psw = nullptr, int pdt = 0,
-                                                            uint32_t L32 = 1) {
+                                                            uint32_t L32 = 1, FillShare fill = FillShare{}) {
+  if (fill_share(fill)) return;
   static_assert(!(FIRST && LOCAL), "the local pass reads the bucketed keys");
   constexpr int R = 1 << BITS;
   constexpr int DPT = R / 256;  // digits per thread in the digit scan
@@ -543,9 +593,10 @@ __global__ __launch_bounds__(256) void seg_plan_kernel(const uint32_t* __restric
 // Per segment: counts of the low digit (keys & (2^BITS - 1)).
 template <int BITS>
 __global__ __launch_bounds__(256) void seg_hist_kernel(const uint32_t* __restrict__ keys, SegTab seg,
-                                                       uint32_t* __restrict__ hist) {
+                                                       uint32_t* __restrict__ hist, FillShare fill) {
   constexpr int R = 1 << BITS;
   __shared__ uint32_t h[R];
+  if (fill_share(fill)) return;
   if (blockIdx.x >= seg.tab[2 * seg.max_segs]) return;
   for (int d = threadIdx.x; d < R; d += 256) h[d] = 0;
   __syncthreads();
@@ -722,112 +773,6 @@ __global__ void row_offsets_kernel(const uint32_t* __restrict__ skeys, const uin
       }
     }
     offs[r] = lo;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Segmented reduction over sorted occurrences (generic lane groups).
-// ---------------------------------------------------------------------------
-template <int VPL>
-struct BwdUnroll {
-  static constexpr int U = VPL >= 8 ? 2 : (VPL >= 4 ? 4 : 8);
-};
-
-// acc += sum over sorted occurrences [i_beg, i_end) (in order) of psw[p] * g[p / L];
-// with want_dot, gpsw[p] = <wv, g[p / L]> for each of them.
-template <typename TW, typename TG, int LPG, int VPL>
-__device__ __forceinline__ void reduce_occurrences(uint32_t i_beg, uint32_t i_end, const uint32_t* __restrict__ svals,
-                                                   const void* __restrict__ psw, int pdt,
-                                                   const TG* __restrict__ g, int64_t D, uint32_t L32,
-                                                   int64_t col0, int glane, const float* wv, bool want_dot,
-                                                   void* __restrict__ gpsw, float* acc,
-                                                   float* __restrict__ dsorted = nullptr) {
-  using GT = GradTraits<TW, TG>;
-  constexpr int EPV = VecTraits<TW>::EPV;
-  constexpr int NE = VPL * EPV;
-  constexpr int NV = GT::NV;
-  constexpr int U = BwdUnroll<VPL * NV>::U;
-  constexpr int VSTRIDE = LPG * EPV;
-  for (uint32_t i0 = i_beg; i0 < i_end; i0 += LPG) {
-    const int n = (int)((i_end - i0) < (uint32_t)LPG ? (i_end - i0) : (uint32_t)LPG);
-    uint32_t my_p = 0, my_b = 0;
-    float my_w = 0.f;
-    if (glane < n) {
-      my_p = svals[i0 + glane];
-      my_b = my_p / L32;
-      my_w = psw ? load_scalar(psw, pdt, my_p) : 1.f;
-    }
-    float my_dot = 0.f;
-    for (int jj = 0; jj < n; jj += U) {
-      uint4 gvec[U][VPL * NV];
-      float w[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        w[u] = 0.f;
-        if (jj + u < n) {
-          const uint32_t b = (uint32_t)bcast_i32<LPG>((int)my_b, jj + u);
-          w[u] = bcast_f32<LPG>(my_w, jj + u);
-          const TG* grow = g + (int64_t)b * D + col0;
-#pragma unroll
-          for (int v = 0; v < VPL; ++v)
-#pragma unroll
-            for (int h = 0; h < NV; ++h) gvec[u][v * NV + h] = ld16(grow + v * VSTRIDE + h * (EPV / NV));
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (jj + u < n) {
-          float f[NE];
-#pragma unroll
-          for (int v = 0; v < VPL; ++v) GT::unpack(&gvec[u][v * NV], f + v * EPV);
-#pragma unroll
-          for (int e = 0; e < NE; ++e) acc[e] = __builtin_fmaf(f[e], w[u], acc[e]);
-          if (want_dot) {
-            float d = 0.f;
-#pragma unroll
-            for (int e = 0; e < NE; ++e) d = __builtin_fmaf(wv[e], f[e], d);
-            d = group_sum<LPG>(d);
-            if (glane == jj + u) my_dot = d;
-          }
-        }
-      }
-    }
-    if (want_dot && glane < n) {
-      if (dsorted != nullptr)
-        dsorted[i0 + glane] = my_dot;  // sorted order, scattered by position later
-      else
-        store_scalar(gpsw, pdt, my_p, my_dot);
-    }
-  }
-}
-
-template <typename TW, int LPG, int VPL>
-__device__ __forceinline__ void load_row_f32(const TW* __restrict__ row, int64_t col0, float* f) {
-  constexpr int EPV = VecTraits<TW>::EPV;
-#pragma unroll
-  for (int v = 0; v < VPL; ++v) VecTraits<TW>::unpack(ld16(row + col0 + v * LPG * EPV), f + v * EPV);
-}
-
-// acc += partial sums of a heavy row [beg, end) in chunk order.
-template <int LPG, int VPL, int EPV>
-__device__ __forceinline__ void add_heavy_partials(uint32_t beg, uint32_t end, const float* __restrict__ partials,
-                                                   int64_t D, int64_t col0, float* acc) {
-  constexpr int VSTRIDE = LPG * EPV;
-  const uint32_t c_first = beg / kHeavyT, c_last = (end - 1) / kHeavyT;
-#pragma unroll 4
-  for (uint32_t c = c_first; c <= c_last; ++c) {
-    const int slot = (c == c_first && beg != c * (uint32_t)kHeavyT) ? 1 : 0;
-    const float* prow = partials + (2 * (int64_t)c + slot) * D + col0;
-#pragma unroll
-    for (int v = 0; v < VPL; ++v) {
-#pragma unroll
-      for (int h = 0; h < EPV; h += 4) {
-        float f[4];
-        VecTraits<float>::unpack(ld16(prow + v * VSTRIDE + h), f);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[v * EPV + h + e] += f[e];
-      }
-    }
   }
 }
 
@@ -2220,8 +2165,27 @@ static BwdLayout bwd_layout(int64_t K, int64_t D, int64_t bags, int64_t L) {
   return l;
 }
 
-// In-place exclusive prefix sum of data[0..n) with data[n] <- total.
+// The sparse plan past small_plan's sizes: 64-lane rows, lookups sorted by the
+// two-level sort, at most a fourth of the rows. Forward + backward, general ->
+// sparse: 64 x 256 into 2^20 x 1024 bf16 531 -> 408 us, 2048 x 128 into 2^20 x
+// 1024 bf16 924 -> 727, 512 x 128 Zipf(1.1) into 2^18 x 1024 bf16 463 -> 255,
+// 1000 x 36 into 2^18 x 512 f32 180 -> 180. Backward alone at half as many
+// lookups as rows: it depends (2^20 x 1024 bf16 868 -> 802, 2^18 x 1024 f32 376
+// -> 405); with as many, the general plan's walk is the faster one (2^18 x 1024
+// f32 438 -> 554); narrow rows it walks four and more a wave (1024 x 64 into
+// 2^18 x 256 bf16 95 -> 112).
+constexpr int64_t kSparseRows = 4;
+static bool sparse_plan(const BwdLayout& l, int lpg, int64_t N, int64_t K) {
+  return lpg == 64 && N > 0 && l.plan.passes == 2 && N * kSparseRows <= K;
+}
+
+// In-place exclusive prefix sum of data[0..n) with data[n] <- total: one block
+// where the data are few (three launches of 4.5 us each otherwise).
 static void device_exclusive_sum(uint32_t* data, int64_t n, uint32_t* parts, hipStream_t st) {
+  if (n <= kScanOneMax) {
+    hipLaunchKernelGGL(scan_one_kernel, dim3(1), dim3(1024), 0, st, data, (int)n);
+    return;
+  }
   const int64_t tiles = cdiv(n, kScanTile);
   hipLaunchKernelGGL(scan_reduce_kernel, dim3((unsigned)tiles), dim3(kScanThreads), 0, st, data, n, parts);
   hipLaunchKernelGGL(scan_parts_kernel, dim3(1), dim3(kScanThreads), 0, st, parts, tiles);
@@ -2268,23 +2232,43 @@ template <int BITS>
 static void two_level_sort(const int64_t* idx, uint32_t* const keys[2], uint32_t* const vals[2], int64_t N, int64_t K,
                            const BwdLayout& l, char* ws, uint32_t* hist, uint32_t* parts, uint32_t* invalid,
                            uint32_t* offs, uint2* meta, const void* psw, int pdt, int64_t L, uint32_t long_min,
-                           uint32_t* long_rows, uint32_t* hot_rows, hipStream_t st) {
+                           uint32_t* long_rows, uint32_t* hot_rows, uint4* fill, size_t fill_n, hipStream_t st) {
   const uint32_t* nvalid = hist + l.nbins;  // the first pass's scan total
-  const dim3 grid((unsigned)l.ntiles), block(256);
-  hipLaunchKernelGGL((radix_hist_kernel<true, BITS>), grid, block, 0, st, idx, (const uint32_t*)nullptr, N,
-                     (const uint32_t*)nullptr, K, BITS, hist, l.ntiles, invalid);
+  const dim3 block(256);
+  // the fill's share of a launch of `blocks` workgroups: pieces [from, to) of 8 parts of it
+  const uint32_t pieces = fill_n > 0 ? fill_pieces(fill_n, 256) : 0u;
+  auto share = [&](int64_t blocks, int from, int to, unsigned* grid) {
+    FillShare f;
+    *grid = (unsigned)blocks;
+    if (pieces == 0) return f;
+    f.p = fill;
+    f.n = fill_n;
+    f.blocks = (uint32_t)blocks;
+    f.first_block = (uint32_t)((blocks + 7) / 8 * 8);
+    f.piece0 = (uint32_t)((uint64_t)(pieces / 8) * from / 8) * 8;
+    const uint32_t last = (uint32_t)((uint64_t)(pieces / 8) * to / 8) * 8;
+    *grid = f.first_block + (last - f.piece0);
+    return f;
+  };
+  unsigned grid;
+  // (shares by what each launch alone takes: the counts, the two scatters, the segment counts)
+  FillShare f = share(l.ntiles, 0, 2, &grid);
+  hipLaunchKernelGGL((radix_hist_kernel<true, BITS>), dim3(grid), block, 0, st, idx, (const uint32_t*)nullptr, N,
+                     (const uint32_t*)nullptr, K, BITS, hist, l.ntiles, invalid, f);
   device_exclusive_sum(hist, l.nbins, parts, st);
-  hipLaunchKernelGGL((radix_scatter_kernel<true, BITS>), grid, block, 0, st, idx, (const uint32_t*)nullptr,
+  f = share(l.ntiles, 2, 5, &grid);
+  hipLaunchKernelGGL((radix_scatter_kernel<true, BITS>), dim3(grid), block, 0, st, idx, (const uint32_t*)nullptr,
                      (const uint32_t*)nullptr, N, (const uint32_t*)nullptr, K, BITS, (const uint32_t*)hist, l.ntiles,
-                     keys[0], vals[0], SegTab{}, (uint2*)nullptr, (const void*)nullptr, 0, 1u);
+                     keys[0], vals[0], SegTab{}, (uint2*)nullptr, (const void*)nullptr, 0, 1u, f);
   uint32_t* tab = (uint32_t*)(ws + l.seg_tab);
   uint32_t* bseg = (uint32_t*)(ws + l.bseg);
   uint32_t* shist = (uint32_t*)(ws + l.seg_hist);
   const SegTab seg{tab, l.max_segs};
   hipLaunchKernelGGL(seg_plan_kernel, dim3(1), dim3(256), 0, st, (const uint32_t*)hist, l.ntiles, (int)l.nbuckets,
                      1 << BITS, nvalid, tab, l.max_segs, bseg, K, offs, meta, l.nmeta);
-  hipLaunchKernelGGL((seg_hist_kernel<BITS>), dim3((unsigned)l.max_segs), dim3(256), 0, st, (const uint32_t*)keys[0],
-                     seg, shist);
+  f = share(l.max_segs, 5, 6, &grid);
+  hipLaunchKernelGGL((seg_hist_kernel<BITS>), dim3(grid), dim3(256), 0, st, (const uint32_t*)keys[0],
+                     seg, shist, f);
   hipLaunchKernelGGL((seg_base_kernel<BITS>), dim3((unsigned)l.nbuckets), dim3(256), 0, st, (const uint32_t*)bseg, K,
                      shist, offs, long_min, long_rows, long_rows != nullptr ? long_rows + K : (uint32_t*)nullptr,
                      (uint32_t)l.hot_min, hot_rows != nullptr ? (uint32_t*)(ws + l.hot_bcnt) : (uint32_t*)nullptr);
@@ -2292,9 +2276,10 @@ static void two_level_sort(const int64_t* idx, uint32_t* const keys[2], uint32_t
     hipLaunchKernelGGL((hot_order_kernel<BITS>), dim3((unsigned)l.nbuckets), dim3(256), 0, st,
                        (const uint32_t*)(ws + l.hot_bcnt), l.nbuckets, (const uint32_t*)offs, K, (uint32_t)l.hot_min,
                        hot_rows, l.hr_max);
-  hipLaunchKernelGGL((radix_scatter_kernel<false, BITS, true>), dim3((unsigned)l.max_segs), block, 0, st,
+  f = share(l.max_segs, 6, 8, &grid);
+  hipLaunchKernelGGL((radix_scatter_kernel<false, BITS, true>), dim3(grid), block, 0, st,
                      (const int64_t*)nullptr, (const uint32_t*)keys[0], (const uint32_t*)vals[0], N, nvalid, K, 0,
-                     (const uint32_t*)shist, (int64_t)0, keys[1], vals[1], seg, meta, psw, pdt, (uint32_t)L);
+                     (const uint32_t*)shist, (int64_t)0, keys[1], vals[1], seg, meta, psw, pdt, (uint32_t)L, f);
 }
 
 // Row-kernel prefetch depth (lookups per row reduced in the row kernel) for
@@ -2596,7 +2581,7 @@ namespace pkm {
 // products (the reductions other than the SGD epilogue use them).
 static int eb_bwd_prepare(int64_t num_rows, int64_t dim, int weight_dtype, const int64_t* indices, const void* psw,
                           int psw_dtype, int64_t bags, int64_t bag_size, void* workspace, size_t workspace_bytes,
-                          bool hot, void* stream) {
+                          bool hot, void* fill, void* stream) {
   GroupCfg c;
   BwdLayout l;
   const int rc = eb_bwd_check("pkm_eb_bwd_prepare", num_rows, dim, weight_dtype, indices, psw, psw_dtype, bags,
@@ -2606,28 +2591,35 @@ static int eb_bwd_prepare(int64_t num_rows, int64_t dim, int weight_dtype, const
   char* ws = (char*)workspace;
   const int64_t K = num_rows, N = bags * bag_size;
   const SortedView v = sorted_view(l, ws);
-  hot = hot && c.lpg == 64 && weight_dtype == PKM_DTYPE_BF16 && hot_rows_enabled(l, dim);
+  const size_t table = (size_t)K * (size_t)dim * (size_t)elem_size(weight_dtype);
+  if (hot && small_plan(N)) {  // (not for the SGD epilogue, which writes every row)
+    const int src = small_sort(indices, N, K, v.keys, v.vals, (uint32_t*)v.nvalid, fill, table, st);
+    return src != PKM_OK ? src : pkm_check_launch("pkm_eb_bwd_prepare");
+  }
+  const bool sparse = hot && sparse_plan(l, c.lpg, N, K);
+  hot = hot && !sparse && c.lpg == 64 && weight_dtype == PKM_DTYPE_BF16 && hot_rows_enabled(l, dim);
   // zeroed state: the out-of-range count, and for the 64-lane row kernels the long-row count, the hot-row
   // state and the zero row
   {
-    const bool rows64 = c.lpg == 64;
+    const bool rows64 = c.lpg == 64 && !sparse;
     hipLaunchKernelGGL(prep_fill_kernel, dim3(rows64 ? grid_for(dim, 256, 64) : 1), dim3(256), 0, st, v.invalid,
                        rows64 && K > 0 ? (uint32_t*)(ws + l.long_rows) + K : (uint32_t*)nullptr,
                        hot ? (uint32_t*)(ws + l.hot_rows) + l.hr_max : (uint32_t*)nullptr,
                        rows64 ? (uint32_t*)(ws + l.zrow) : (uint32_t*)nullptr, rows64 ? dim : (int64_t)0);
   }
-  uint2* meta = c.lpg == 64 ? (uint2*)(ws + l.meta) : nullptr;  // read by the 64-lane row kernels
+  uint2* meta = c.lpg == 64 && !sparse ? (uint2*)(ws + l.meta) : nullptr;  // read by the 64-lane row kernels
   if (N > 0 && l.plan.passes == 2) {
     // 1-2. stable sort of (row, position) by bucketing and local passes, with the row offsets, the metadata and
     // the 64-lane row kernel's long-row list
     uint32_t* keys[2] = {(uint32_t*)(ws + l.keys0), (uint32_t*)(ws + l.keys1)};
     uint32_t* vals[2] = {(uint32_t*)(ws + l.vals0), (uint32_t*)(ws + l.vals1)};
-    uint32_t* long_rows = c.lpg == 64 ? (uint32_t*)(ws + l.long_rows) : nullptr;
+    uint32_t* long_rows = c.lpg == 64 && !sparse ? (uint32_t*)(ws + l.long_rows) : nullptr;
     uint32_t* hot_rows = hot ? (uint32_t*)(ws + l.hot_rows) : nullptr;
     const uint32_t long_min = (uint32_t)(2 * rows_prefetch_of(c.vpl, N, K));
 #define PKM_TWO_LEVEL(B_)                                                                                      \
   two_level_sort<B_>(indices, keys, vals, N, K, l, ws, v.hist, v.parts, v.invalid, v.offs, meta, psw, psw_dtype, \
-                     bag_size, long_min, long_rows, hot_rows, st)
+                     bag_size, long_min, long_rows, hot_rows, (uint4*)(sparse ? fill : nullptr),           \
+                     sparse && fill != nullptr ? table / 16 : 0, st)
     switch (l.plan.bits) {
       case 8:
         PKM_TWO_LEVEL(8);
@@ -2666,6 +2658,7 @@ static int eb_bwd_prepare(int64_t num_rows, int64_t dim, int weight_dtype, const
   } else {
     hipLaunchKernelGGL(fill_u32_kernel, dim3(grid_for(K + 1, 256, 4096)), dim3(256), 0, st, v.offs, 0u, K + 1);
   }
+  if (sparse) return pkm_check_launch("pkm_eb_bwd_prepare");
   // 3. metadata and the row kernel's lists
   bool ok;
   if (weight_dtype == PKM_DTYPE_F32)
@@ -2686,13 +2679,15 @@ extern "C" int pkm_eb_bwd_prepare(int64_t num_rows, int64_t dim, int weight_dtyp
                                   const void* psw, int psw_dtype, int64_t bags, int64_t bag_size, void* workspace,
                                   size_t workspace_bytes, void* stream) {
   return eb_bwd_prepare(num_rows, dim, weight_dtype, indices, psw, psw_dtype, bags, bag_size, workspace,
-                        workspace_bytes, true, stream);
+                        workspace_bytes, true, nullptr, stream);
 }
 
 namespace pkm {
 // The reduction on a prepared workspace; acc: grad_weight holds a gradient
 // that the rows' sums are added to (rows without lookups keep it).
-static int eb_bwd_reduce(const char* fn, bool acc, const void* weight, int64_t num_rows, int64_t dim,
+// sort: the workspace is prepared here first (by the sparse plan beside the
+// table gradient's zeros).
+static int eb_bwd_reduce(const char* fn, bool acc, bool sort, const void* weight, int64_t num_rows, int64_t dim,
                          int weight_dtype, const int64_t* indices, const void* psw, int psw_dtype,
                          const void* grad_out, int grad_dtype, int64_t bags, int64_t bag_size, void* grad_weight,
                          void* grad_psw, void* workspace, size_t workspace_bytes, void* stream) {
@@ -2717,6 +2712,27 @@ static int eb_bwd_reduce(const char* fn, bool acc, const void* weight, int64_t n
   const SortedView v = sorted_view(l, ws);
   void* gpsw = psw != nullptr ? grad_psw : nullptr;
   const int64_t K = num_rows;
+  const bool small = small_plan(N);
+  if (small || sparse_plan(l, c.lpg, N, K)) {
+    // the zeros come with the sort where it runs here
+    void* fill = acc ? nullptr : grad_weight;
+    const int src = sort ? eb_bwd_prepare(num_rows, dim, weight_dtype, indices, psw, psw_dtype, bags, bag_size,
+                                          workspace, workspace_bytes, true, fill, stream)
+                    : fill != nullptr
+                        ? sparse_fill(fill, (size_t)K * (size_t)dim * (size_t)elem_size(weight_dtype), st)
+                        : PKM_OK;
+    if (src != PKM_OK) return src;
+    PKM_REQUIRE(sparse_reduce(c, weight_dtype, grad_dtype, acc, weight, K, dim, psw, psw_dtype, grad_out, bag_size,
+                              v.keys, v.vals, v.nvalid, N, small ? nullptr : v.invalid, (float*)(ws + l.partials),
+                              grad_weight, gpsw, st),
+                PKM_ERR_UNSUPPORTED, "%s: no kernel for lpg=%d vpl=%d", fn, c.lpg, c.vpl);
+    return pkm_check_launch(fn);
+  }
+  if (sort) {
+    const int src = eb_bwd_prepare(num_rows, dim, weight_dtype, indices, psw, psw_dtype, bags, bag_size, workspace,
+                                   workspace_bytes, true, nullptr, stream);
+    if (src != PKM_OK) return src;
+  }
   // 4-5. heavy-row chunk partials, then every row once, then the psw-gradients to their positions
   bool ok;
 #define PKM_REDUCE(TW_, TG_)                                                                                    \
@@ -2749,7 +2765,7 @@ extern "C" int pkm_eb_bwd_prepared(const void* weight, int64_t num_rows, int64_t
                                    const int64_t* indices, const void* psw, int psw_dtype, const void* grad_out,
                                    int grad_dtype, int64_t bags, int64_t bag_size, void* grad_weight, void* grad_psw,
                                    void* workspace, size_t workspace_bytes, void* stream) {
-  return eb_bwd_reduce("pkm_eb_bwd_prepared", false, weight, num_rows, dim, weight_dtype, indices, psw, psw_dtype,
+  return eb_bwd_reduce("pkm_eb_bwd_prepared", false, false, weight, num_rows, dim, weight_dtype, indices, psw, psw_dtype,
                        grad_out, grad_dtype, bags, bag_size, grad_weight, grad_psw, workspace, workspace_bytes,
                        stream);
 }
@@ -2762,10 +2778,7 @@ extern "C" int pkm_eb_bwd_accumulate(const void* weight, int64_t num_rows, int64
               "pkm_eb_bwd_accumulate: dim %lld, weight dtype %d, grad dtype %d not supported (grad_out in the "
               "table's dtype, rows of 64 16-byte vectors or more)",
               (long long)dim, weight_dtype, grad_dtype);
-  const int rc = pkm_eb_bwd_prepare(num_rows, dim, weight_dtype, indices, psw, psw_dtype, bags, bag_size, workspace,
-                                    workspace_bytes, stream);
-  if (rc != PKM_OK) return rc;
-  return eb_bwd_reduce("pkm_eb_bwd_accumulate", true, weight, num_rows, dim, weight_dtype, indices, psw, psw_dtype,
+  return eb_bwd_reduce("pkm_eb_bwd_accumulate", true, true, weight, num_rows, dim, weight_dtype, indices, psw, psw_dtype,
                        grad_out, grad_dtype, bags, bag_size, grad_weight, grad_psw, workspace, workspace_bytes,
                        stream);
 }
@@ -2778,11 +2791,9 @@ extern "C" int pkm_eb_bwd(const void* weight, int64_t num_rows, int64_t dim, int
               PKM_ERR_UNSUPPORTED,
               "pkm_eb_bwd: grad_out dtype %d with weight dtype %d (supported: the same dtype, or a float32 "
               "grad_out for a 16-bit table)", grad_dtype, weight_dtype);
-  const int rc = pkm_eb_bwd_prepare(num_rows, dim, weight_dtype, indices, psw, psw_dtype, bags, bag_size, workspace,
-                                    workspace_bytes, stream);
-  if (rc != PKM_OK) return rc;
-  return pkm_eb_bwd_prepared(weight, num_rows, dim, weight_dtype, indices, psw, psw_dtype, grad_out, grad_dtype, bags,
-                             bag_size, grad_weight, grad_psw, workspace, workspace_bytes, stream);
+  return eb_bwd_reduce("pkm_eb_bwd", false, true, weight, num_rows, dim, weight_dtype, indices, psw, psw_dtype,
+                       grad_out, grad_dtype, bags, bag_size, grad_weight, grad_psw, workspace, workspace_bytes,
+                       stream);
 }
 
 extern "C" int pkm_eb_bwd_sgd(const void* values, int64_t num_rows, int64_t dim, int dtype, const int64_t* indices,
@@ -2812,7 +2823,7 @@ extern "C" int pkm_eb_bwd_sgd(const void* values, int64_t num_rows, int64_t dim,
   PKM_REQUIRE(((uintptr_t)values | (uintptr_t)grad_out | (uintptr_t)new_values | (uintptr_t)scaled_grad) % 16 == 0,
               PKM_ERR_INVALID_ARGUMENT, "pkm_eb_bwd_sgd: values, grad_out and outputs must be 16-byte aligned");
   rc = eb_bwd_prepare(num_rows, dim, dtype, indices, psw, psw_dtype, bags, bag_size, workspace, workspace_bytes,
-                      false, stream);
+                      false, nullptr, stream);
   if (rc != PKM_OK) return rc;
   hipStream_t st = (hipStream_t)stream;
   char* ws = (char*)workspace;

@@ -307,6 +307,7 @@ struct GroupCfg {
   int64_t slices;
 };
 bool choose_group_cfg(int64_t D, int epv, bool single_slice, GroupCfg* c);
+int elem_size(int dt);  // bytes of an element of dtype code dt
 
 // ---------------------------------------------------------------------------
 // Error reporting (host side), defined in capi.hip.

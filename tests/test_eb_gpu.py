@@ -595,6 +595,53 @@ def test_backward_hot_rows_chunk_densities(L, device):
     assert torch.equal(gW, gW2) and torch.equal(gp, gp2)
 
 
+# The sparse plan's edges: the one-workgroup sort's last size and the two-level
+# sort after it, the last row count it takes and one row fewer (the general
+# plan), one and two keys of 8-bit digits; runs of 1 to 300 lookups across
+# windows, waves and heavy chunks, a run of the first and of the last row,
+# out-of-range lookups; weighted, unweighted, a float32 gradient of a 16-bit
+# table. Also prepared ahead and accumulating, bit for bit.
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 256), (torch.float32, 2048), (torch.bfloat16, 512),
+                                     (torch.bfloat16, 4096), (torch.float16, 1024), (torch.bfloat16, 64),
+                                     (torch.bfloat16, 256)], ids=str)
+@pytest.mark.parametrize("B,L,K", [(3, 5, 70), (80, 128, 200), (80, 128, 70000), (10241, 1, 40964), (10241, 1, 40963),
+                                   (41, 301, 70001)])
+def test_backward_sparse_plan(B, L, K, D, dtype, device):
+    from modelos_amd import embedding_bag as eb
+
+    W, _, p, g = eb_inputs(B, L, K, D, dtype, seed=81 + D)
+    gen = torch.Generator().manual_seed(82)
+    flat = torch.randint(0, K, (B * L,), generator=gen)
+    pos = torch.randperm(B * L, generator=gen)
+    at = 0
+    for row, n in ((0, 3), (1, 16), (2, 17), (3, 64), (4, 65), (5, 256), (6, 257), (7, 300), (K - 1, 40), (-1, 5), (K, 4)):
+        if at + n <= B * L // 2:
+            flat[pos[at:at + n]] = row
+            at += n
+    idx = flat.view(B, L)
+    args = _dev(idx, W, p, g, device=device)
+    eW, ep = ref.eb_backward(idx, W, p, g)
+    cW, cp = ref.eb_backward(idx, W.abs(), p.abs(), g.abs())
+    gW, gp = eb.eb_backward(*args)
+    assert_rel_close(gW, eW, REL_TOL[dtype], "grad_weight", cond=cW)
+    assert_rel_close(gp, ep, REL_TOL[dtype], "grad_psw", cond=cp)
+    assert (gp.cpu()[(idx < 0) | (idx >= K)] == 0).all()
+    pW, pp = eb.eb_backward(*args, prepared=eb.eb_backward_prepare(args[0], args[1], args[2]))
+    assert torch.equal(pW, gW) and torch.equal(pp, gp)
+    pending = torch.randn((K, D), generator=gen).to(dtype).to(device)
+    res = eb.eb_backward_into(*args, pending.clone())
+    if res is not None:  # (64-lane rows)
+        assert torch.equal(res[0], pending + gW) and torch.equal(res[1], gp)
+    uW, up = eb.eb_backward(args[0], args[1], None, args[3])
+    assert up is None
+    assert_rel_close(uW, ref.eb_backward(idx, W, None, g)[0], REL_TOL[dtype], "unweighted",
+                     cond=ref.eb_backward(idx, W.abs(), None, g.abs())[0])
+    if dtype != torch.float32:
+        wW, wp = eb.eb_backward(args[0], args[1], args[2], args[3].float())
+        assert_rel_close(wW, eW, REL_TOL[dtype], "float32 gradient", cond=cW)
+        assert_rel_close(wp, ep, REL_TOL[dtype], "float32 gradient, psw", cond=cp)
+
+
 # Rows longer than the row kernel's prefetch but below the heavy threshold
 # (5..250 lookups), packed into the first 64-row windows, beside two heavy rows
 # and uniform rows: with more than 3 lookups per row on average (the 8-slot
