@@ -295,15 +295,19 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_fused_kernel(const T* __restr
 }
 
 // dw[j] = sum over the row blocks b (in order) of part[b, j]: 64 columns per
-// block, the partials split over 4 thread slices (each summing a contiguous
-// range of blocks, loads kept in flight), the slices added in order.
+// block, the partials split over 16 waves (each summing a contiguous range of
+// blocks, loads kept in flight), the waves' sums added in order. 64 blocks for
+// 4096 columns: what bounds it is a wave's chain of loads (1024 partial rows: 4
+// waves a block 11.2 us, 16 5.0).
+constexpr int kNormSlices = 16;
 template <typename T>
-__global__ __launch_bounds__(256) void rmsnorm_bwd_dw_reduce_kernel(const float* __restrict__ part, int64_t nrb,
-                                                                    int D, T* __restrict__ dw) {
-  __shared__ float ps[4][64];
+__global__ __launch_bounds__(64 * kNormSlices) void rmsnorm_bwd_dw_reduce_kernel(const float* __restrict__ part,
+                                                                                 int64_t nrb, int D,
+                                                                                 T* __restrict__ dw) {
+  __shared__ float ps[kNormSlices][64];
   const int jl = threadIdx.x & 63, sl = threadIdx.x >> 6;
   const int j = blockIdx.x * 64 + jl;
-  const int64_t per = (nrb + 3) / 4;
+  const int64_t per = (nrb + kNormSlices - 1) / kNormSlices;
   const int64_t b0 = sl * per, b1 = b0 + per < nrb ? b0 + per : nrb;
   float s = 0.f;
   if (j < D) {
@@ -320,7 +324,9 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_dw_reduce_kernel(const float*
   ps[sl][jl] = s;
   __syncthreads();
   if (sl == 0 && j < D) {
-    const float t = ((ps[0][jl] + ps[1][jl]) + ps[2][jl]) + ps[3][jl];
+    float t = ps[0][jl];
+#pragma unroll
+    for (int k = 1; k < kNormSlices; ++k) t += ps[k][jl];
     if (sizeof(T) == 4)
       ((float*)dw)[j] = t;
     else
@@ -390,10 +396,10 @@ extern "C" int pkm_rmsnorm_bwd(const void* dy, const void* x, const void* weight
   if (rows == 0) {  // dweight = 0 (a reduction over no partials)
     const dim3 rgrid((unsigned)((D + 63) / 64));
     if (dtype == PKM_DTYPE_BF16)
-      hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<bf16_t>), rgrid, dim3(256), 0, st, (const float*)nullptr,
+      hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<bf16_t>), rgrid, dim3(64 * kNormSlices), 0, st, (const float*)nullptr,
                          (int64_t)0, D, (bf16_t*)dweight);
     else
-      hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<float>), rgrid, dim3(256), 0, st, (const float*)nullptr,
+      hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<float>), rgrid, dim3(64 * kNormSlices), 0, st, (const float*)nullptr,
                          (int64_t)0, D, (float*)dweight);
     return pkm_check_launch("pkm_rmsnorm_bwd");
   }
@@ -418,12 +424,12 @@ extern "C" int pkm_rmsnorm_bwd(const void* dy, const void* x, const void* weight
     if (dtype == PKM_DTYPE_BF16) {
       hipLaunchKernelGGL((rmsnorm_bwd_fused_kernel<bf16_t>), fgrid, dim3(256), 0, st, (const bf16_t*)dy,
                          (const bf16_t*)x, (const bf16_t*)weight, rstd, rows, D, (bf16_t*)dx, part);
-      hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<bf16_t>), rgrid, dim3(256), 0, st, (const float*)part, fnrb,
+      hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<bf16_t>), rgrid, dim3(64 * kNormSlices), 0, st, (const float*)part, fnrb,
                          D, (bf16_t*)dweight);
     } else {
       hipLaunchKernelGGL((rmsnorm_bwd_fused_kernel<float>), fgrid, dim3(256), 0, st, (const float*)dy,
                          (const float*)x, (const float*)weight, rstd, rows, D, (float*)dx, part);
-      hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<float>), rgrid, dim3(256), 0, st, (const float*)part, fnrb, D,
+      hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<float>), rgrid, dim3(64 * kNormSlices), 0, st, (const float*)part, fnrb, D,
                          (float*)dweight);
     }
   } else if (dtype == PKM_DTYPE_BF16) {
@@ -431,14 +437,14 @@ extern "C" int pkm_rmsnorm_bwd(const void* dy, const void* x, const void* weight
                        (const bf16_t*)x, (const bf16_t*)weight, rstd, rows, D, (bf16_t*)dx);
     hipLaunchKernelGGL((rmsnorm_bwd_dw_partial_kernel<bf16_t>), pgrid, dim3(256), 0, st, (const bf16_t*)dy,
                        (const bf16_t*)x, rstd, rows, D, part);
-    hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<bf16_t>), rgrid, dim3(256), 0, st, (const float*)part, nrb, D,
+    hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<bf16_t>), rgrid, dim3(64 * kNormSlices), 0, st, (const float*)part, nrb, D,
                        (bf16_t*)dweight);
   } else {
     hipLaunchKernelGGL((rmsnorm_bwd_dx_kernel<float, 0>), grid, dim3(256), 0, st, (const float*)dy,
                        (const float*)x, (const float*)weight, rstd, rows, D, (float*)dx);
     hipLaunchKernelGGL((rmsnorm_bwd_dw_partial_kernel<float>), pgrid, dim3(256), 0, st, (const float*)dy,
                        (const float*)x, rstd, rows, D, part);
-    hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<float>), rgrid, dim3(256), 0, st, (const float*)part, nrb, D,
+    hipLaunchKernelGGL((rmsnorm_bwd_dw_reduce_kernel<float>), rgrid, dim3(64 * kNormSlices), 0, st, (const float*)part, nrb, D,
                        (float*)dweight);
   }
   return pkm_check_launch("pkm_rmsnorm_bwd");
