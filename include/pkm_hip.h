@@ -509,6 +509,22 @@ int pkm_swilu_bwd(const void* dh, const void* e, const void* s, int64_t n, int d
                   void* stream);
 
 /*
+ * The elementwise end of an idw score gradient, float32: out = 2 (products - x
+ * * row_factors[b, t]) over batches x rows rows of dim. products [batches, rows,
+ * dim], row_factors [batches, rows]; x and out [rows, batches, dim] with
+ * row_major (queries), else [batches, rows, dim] (keys). Every step rounded, no
+ * contraction. dim a multiple of 4, buffers 16-byte aligned.
+ *
+ * Replaces part of the autograd of cdist (fwpkm/fwpkm.py:853-869).
+ */
+int pkm_idw_grad_finish(const float* products, const float* x, const float* row_factors, int64_t batches,
+                        int64_t rows, int64_t dim, int row_major, float* out, void* stream);
+
+/* out[b, t] = sum of squares of row t of batch b of x (layouts as above), float32. */
+int pkm_row_sumsq(const float* x, int64_t batches, int64_t rows, int64_t dim, int row_major, float* out,
+                  void* stream);
+
+/*
  * A Linear over a few rows: y[i, o] = bf16(sum_k x[i, k] * weight[o, k] + bias[o]),
  * float32 sums, one rounding. x [rows, in_features], weight [out_features,
  * in_features], bias [out_features] or NULL, y [rows, out_features]; bfloat16,

@@ -29,7 +29,7 @@ import torch
 
 from .. import _lib
 from ..embedding_bag import _aligned, _require_device
-from ..product_keys import SCORE_TYPES, share_distance_products
+from ..product_keys import SCORE_TYPES, _idw_finish, _row_sumsq, share_distance_products
 
 ME_MAX_N_KEYS = 1024
 _DTYPES = (torch.float32, torch.bfloat16, torch.float16)
@@ -68,8 +68,8 @@ class _AddrKeyGrad(torch.autograd.Function):
         if idw:
             # the reference path's mm-based distance operands (|q|^2 + |k|^2 - 2 <q, k>)
             dots = torch.bmm(qb, kf.transpose(1, 2).contiguous())
-            qq = (qb * qb).sum(-1).contiguous()
-            kk = (kf * kf).sum(-1).contiguous()
+            qq = _row_sumsq(query.detach().float().reshape(tokens, 2 * heads, half), True)
+            kk = _row_sumsq(kf, False)
             if share_with is not None:
                 # the retrieval's backward needs the same products of the same operands
                 share_distance_products(share_with, dots, qq, kk)
@@ -85,7 +85,7 @@ class _AddrKeyGrad(torch.autograd.Function):
                   _lib.ptr(pbar), _lib.ptr(cs), _lib.ptr(ws), ws.numel(), _lib.stream_of(dev))
         g = torch.bmm(coef.transpose(1, 2), qb)
         if idw:
-            g = 2.0 * (g - kf * cs[:, :, None])
+            g = _idw_finish(g, kf, cs, False)
         ctx.heads, ctx.topk, ctx.weight, ctx.score_type = heads, topk, float(weight), score_type
         ctx.query_shape, ctx.query_dtype, ctx.keys_dtype = query.shape, query.dtype, keys.dtype
         # idw: the forward-time key values (kf is a copy when the keys are not float32; the

@@ -221,6 +221,39 @@ def _idw_grad_coef(dS, qq, kk, dots):
     return U, rs, cs
 
 
+def _vector_rows(*tensors) -> bool:
+    """Contiguous float32 tensors of 16-byte aligned rows of whole vectors."""
+    return all(t.dtype == torch.float32 and t.is_contiguous() and t.shape[-1] % 4 == 0 and t.data_ptr() % 16 == 0
+               for t in tensors)
+
+
+def _row_sumsq(x, row_major):
+    """Sums of squares [batches, rows] of x's rows: x [batches, rows, dim], or
+    with row_major [rows, batches, dim]."""
+    if not _vector_rows(x):
+        s = (x * x).sum(-1)
+        return (s.t() if row_major else s).contiguous()
+    B, T = (x.shape[1], x.shape[0]) if row_major else x.shape[:2]
+    out = torch.empty((B, T), dtype=torch.float32, device=x.device)
+    _lib.call("pkm_row_sumsq", _lib.ptr(x), B, T, x.shape[2], int(row_major), _lib.ptr(out), _lib.stream_of(x.device))
+    return out
+
+
+def _idw_finish(products, x, factors, row_major):
+    """2 (products - x * factors): products [batches, rows, dim], factors
+    [batches, rows]; x and the result [batches, rows, dim], or with row_major
+    [rows, batches, dim]."""
+    if not _vector_rows(products, x):
+        f = factors[:, :, None]
+        return (2.0 * (products.transpose(0, 1) - x * f.transpose(0, 1)) if row_major
+                else 2.0 * (products - x * f))
+    out = torch.empty_like(x)
+    _lib.call("pkm_idw_grad_finish", _lib.ptr(products), _lib.ptr(x), _lib.ptr(factors.contiguous()),
+              products.shape[0], products.shape[1], products.shape[2], int(row_major), _lib.ptr(out),
+              _lib.stream_of(x.device))
+    return out
+
+
 def share_distance_products(sub_scores: torch.Tensor, dots: torch.Tensor, qq: torch.Tensor, kk: torch.Tensor) -> None:
     """Hands the float32 distance operands of an idw retrieval (dots [2 heads,
     tokens, n] = <q_t, k_j>, qq [2 heads, tokens], kk [2 heads, n], taken from
@@ -275,9 +308,16 @@ def _grads_from_dense(query, keys, dS, heads, n, score_type, keys_fwd=None, shar
             U = torch.where(d2 > 0, D.float() / (1e-3 + d2.clamp_min(0.0)), torch.zeros_like(d2))
             rs, cs = U.sum(-1), U.sum(1)
         else:
-            # the same U and its row and column sums in one pass (pkm_idw_grad_coef)
-            qq, kk = (shared[1], shared[2]) if use_shared else ((q32 * q32).sum(-1), (kf * kf).sum(-1))
+            # the same U and its row and column sums in one pass (pkm_idw_grad_coef), and the ends of both
+            # gradients in one pass each, the queries' in their own layout
+            q_rows = query.reshape(N, heads * 2, half).float().contiguous()
+            kf = kf.contiguous()
+            qq, kk = (shared[1], shared[2]) if use_shared else (_row_sumsq(q_rows, True), _row_sumsq(kf, False))
             U, rs, cs = _idw_grad_coef(D, qq, kk, dots)
+            dq = _idw_finish(torch.bmm(U, kf), q_rows, rs, True)
+            # float32 operands: the transposed view goes to the GEMM as it is
+            dk = _idw_finish(torch.bmm(U.transpose(1, 2), q32), kf, cs, False)
+            return dq.reshape(N, heads, 2 * half), dk.reshape(keys.shape)
         dqh = 2.0 * (torch.bmm(U, kf) - q32 * rs[:, :, None])
         # float32 operands: the transposed view goes to the GEMM as it is
         dk = 2.0 * (torch.bmm(U.transpose(1, 2), q32) - kf * cs[:, :, None])
