@@ -1591,7 +1591,9 @@ __host__ inline size_t lds_bytes(int half) {
 
 }  // namespace stream
 
-// Lanes per row of the cartesian kernel: 8 in bulk; 32 up to 8192 rows, where
+// Lanes per row of the cartesian kernel: 8 in bulk, 16 for knn > 32 (280 pairs a
+// row at knn 64: scoring + cartesian of 65536 rows 573 -> 545 us; knn 32, 131072
+// rows, 287 -> 304); 32 up to 8192 rows, where
 // the row's serial chain is what it takes (knn 32, up to 4096 rows: scoring +
 // cartesian 2 to 4 us less; knn 64, 4096 rows 75 -> 63 us, 8192 rows 102 ->
 // 95; 16384 rows of knn 32 72 -> 80).
@@ -1641,8 +1643,9 @@ template <typename TIN>
 static int launch_cartesian(int64_t Ntok, int H, int n, int knn, int lds_max, void* out_scores, int64_t* out_idx,
                             hipStream_t st) {
   const int64_t rows = Ntok * H;
-  return rows <= kCartWideRows ? launch_cartesian_lpr<TIN, 32>(rows, n, knn, lds_max, out_scores, out_idx, st)
-                               : launch_cartesian_lpr<TIN, 8>(rows, n, knn, lds_max, out_scores, out_idx, st);
+  if (rows <= kCartWideRows) return launch_cartesian_lpr<TIN, 32>(rows, n, knn, lds_max, out_scores, out_idx, st);
+  return knn > 32 ? launch_cartesian_lpr<TIN, 16>(rows, n, knn, lds_max, out_scores, out_idx, st)
+                  : launch_cartesian_lpr<TIN, 8>(rows, n, knn, lds_max, out_scores, out_idx, st);
 }
 
 template <typename TIN, int IDW, int TM, int KSC>
