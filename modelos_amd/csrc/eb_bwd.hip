@@ -206,53 +206,42 @@ __global__ __launch_bounds__(256) void scan_reduce_kernel(const uint32_t* __rest
 }
 
 // One block: in-place exclusive prefix sum of data[0..n), data[n] <- the total,
-// 8192 words a step, the next step's loaded while this one's are summed.
-constexpr int64_t kScanOneMax = 16384;  // (two steps: 9.8 us)
+// n <= kScanOneMax. Backward of 100000 lookups into 2^14 x 256 bf16 (6400 words)
+// 70.8 -> 69.4 us against the three launches of the tiled sum, of 50000 64.4 ->
+// 61.3; a second step of 8192 words costs more than they do (200000 lookups,
+// 12544 words: 82.7 -> 86.3).
+constexpr int64_t kScanOneMax = 8192;
 __global__ __launch_bounds__(1024) void scan_one_kernel(uint32_t* __restrict__ data, int n) {
-  __shared__ uint32_t wtot[2][16];
+  __shared__ uint32_t wtot[16];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  uint32_t carry = 0;
-  uint32_t next[8];
-  auto load = [&](int base) {
+  const int p0 = (int)threadIdx.x * 8;
+  uint32_t v[8], s = 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int p = base + (int)threadIdx.x * 8 + i;
-      next[i] = p < n ? data[p] : 0u;
-    }
-  };
-  load(0);
-#pragma unroll 1
-  for (int base = 0, k = 0; base < n; base += 8192, k ^= 1) {
-    uint32_t v[8], s = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      v[i] = next[i];
-      s += v[i];
-    }
-    load(base + 8192);
-    uint32_t x = s;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t y = (uint32_t)__shfl_up((int)x, o);
-      if (lane >= o) x += y;
-    }
-    if (lane == 63) wtot[k][w] = x;
-    __syncthreads();  // (two buffers: the next step's totals don't meet this one's readers)
-    uint32_t run = carry + x - s;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const uint32_t t = wtot[k][i];
-      run += i < w ? t : 0u;
-      carry += t;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int p = base + (int)threadIdx.x * 8 + i;
-      if (p < n) data[p] = run;
-      run += v[i];
-    }
+  for (int i = 0; i < 8; ++i) {
+    v[i] = p0 + i < n ? data[p0 + i] : 0u;
+    s += v[i];
   }
-  if (threadIdx.x == 0) data[n] = carry;
+  uint32_t x = s;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = (uint32_t)__shfl_up((int)x, o);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) wtot[w] = x;
+  __syncthreads();
+  uint32_t run = x - s, total = 0;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const uint32_t t = wtot[i];
+    run += i < w ? t : 0u;
+    total += t;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (p0 + i < n) data[p0 + i] = run;
+    run += v[i];
+  }
+  if (threadIdx.x == 0) data[n] = total;
 }
 
 // Single block: exclusive prefix sum of the per-tile sums, in place.
@@ -2180,7 +2169,7 @@ static bool sparse_plan(const BwdLayout& l, int lpg, int64_t N, int64_t K) {
 }
 
 // In-place exclusive prefix sum of data[0..n) with data[n] <- total: one block
-// where the data are few (three launches of 4.5 us each otherwise).
+// where the data are few.
 static void device_exclusive_sum(uint32_t* data, int64_t n, uint32_t* parts, hipStream_t st) {
   if (n <= kScanOneMax) {
     hipLaunchKernelGGL(scan_one_kernel, dim3(1), dim3(1024), 0, st, data, (int)n);

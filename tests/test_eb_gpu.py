@@ -642,6 +642,21 @@ def test_backward_sparse_plan(B, L, K, D, dtype, device):
         assert_rel_close(wp, ep, REL_TOL[dtype], "float32 gradient, psw", cond=cp)
 
 
+# The digit counts' prefix sum (256 words a tile of 4096 lookups): one block up
+# to 8192 words, three launches past it; one and two digits, and few words.
+@pytest.mark.parametrize("B,L,K", [(10241, 1, 40000), (1024, 128, 60000), (131073, 1, 60000), (1024, 128, 250)])
+def test_backward_digit_scan_sizes(B, L, K, device):
+    from modelos_amd import embedding_bag as eb
+
+    W, idx, p, g = eb_inputs(B, L, K, 8, torch.float32, seed=83)
+    idx.view(-1)[::1001] = -1
+    gW, gp = eb.eb_backward(*_dev(idx, W, p, g, device=device))
+    eW, ep = ref.eb_backward(idx, W, p, g)
+    cW, cp = ref.eb_backward(idx, W.abs(), p.abs(), g.abs())
+    assert_rel_close(gW, eW, REL_TOL[torch.float32], "grad_weight", cond=cW)
+    assert_rel_close(gp, ep, REL_TOL[torch.float32], "grad_psw", cond=cp)
+
+
 # Rows longer than the row kernel's prefetch but below the heavy threshold
 # (5..250 lookups), packed into the first 64-row windows, beside two heavy rows
 # and uniform rows: with more than 3 lookups per row on average (the 8-slot
