@@ -191,11 +191,18 @@ __global__ __launch_bounds__(256) void eb_fwd_kernel(const TW* __restrict__ W, i
 // 256-byte slices 635 us, 1 KB slices 648 us, 128-byte slices 670 us. With
 // fewer bags every slice is in flight at once and slicing only scatters the
 // reads: one bag a wave, slices fastest (4096 bags x 128, 2^18 x 512: 77 us,
-// 83 us sliced; 500 x 500, 2^16 x 2048: 142 us, 152 us sliced).
+// 83 us sliced; 500 x 500, 2^16 x 2048: 142 us, 152 us sliced). There the
+// layout is nearly the replaced kernel's and so is the time: float32 rows of 1
+// to 16 KB, 512 to 4096 bags of 8 to 512 lookups, 0.95 to 1.26 times its speed;
+// 16-bit rows of 1 KB the same, with 4096 to 8191 bags of 30 lookups and more
+// 1 to 5 % behind it (4096 x 64, 2^16 x 512: 37.3 -> 38.7 us).
 //
 // Row numbers and weights are held 16 to a register in each 16-lane row and
 // broadcast by DPP; the next 16 are loaded a step ahead. Absent lookups read a
-// line of zeros, with weight zero: no load is conditional.
+// line of zeros, with weight zero: no load is conditional. 16 lookups a step,
+// a last one of at most 8 by itself: all steps full, a bag of 8 paid for 16
+// (4096 x 8, 2^14 x 1024 bf16: replaced kernel 12.1 us, full steps 13.5, so
+// 12.2; 512 x 8, 2^16 x 512 f32: 3.2, 3.2, 2.8).
 //
 // NW > 1 where the tasks alone leave the chip idle: 16 lookups each in turn,
 // the waves' float32 sums added in wave order through LDS (8 bags x 256: one
@@ -268,13 +275,23 @@ __global__ __launch_bounds__(64 * kGatherMaxNW) void eb_gather_kernel(const TW* 
     }
   };
   fetch(kGatherLanes * q);
-  for (int64_t j0 = kGatherLanes * q; j0 < L; j0 += step) {
+  int64_t j0 = kGatherLanes * q;
+  uint32_t r;
+  float w;
+  auto take = [&] {
     const bool ok = r_next >= 0 && r_next < K;
-    const uint32_t r = ok ? (uint32_t)r_next : 0xFFFFFFFFu;
-    const float w = ok ? w_next : 0.f;
+    r = ok ? (uint32_t)r_next : 0xFFFFFFFFu;
+    w = ok ? w_next : 0.f;
+  };
+  for (; j0 + 8 < L; j0 += step) {
+    take();
     fetch(j0 + step);
     gather8<TW, 0>(base, row_bytes, r, w, zero, acc, std::make_integer_sequence<int, 8>{});
     gather8<TW, 8>(base, row_bytes, r, w, zero, acc, std::make_integer_sequence<int, 8>{});
+  }
+  if (j0 < L) {  // a last step of at most 8
+    take();
+    gather8<TW, 0>(base, row_bytes, r, w, zero, acc, std::make_integer_sequence<int, 8>{});
   }
   if (NW > 1) {
     float* p = gather_part + (int)threadIdx.x * EPV;

@@ -105,6 +105,27 @@ def test_forward_gather_layouts(B, L, nvec, dtype, device):
     assert_rel_close(out, expect, REL_TOL[dtype], f"forward {dtype} {B,L,D}", cond=cond)
 
 
+# A step of the gather takes 16 lookups, a last one of at most 8 half of it:
+# both sides of each line, with the lookups of a bag in one wave (2048 bags) and
+# shared by several (2 bags). Row 0 holds infinities and is not looked up.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("L", [7, 8, 9, 15, 16, 17, 24, 25, 40, 41, 264, 265])
+@pytest.mark.parametrize("B,nvec", [(2, 16), (2, 64), (2048, 32), (2048, 64)])
+def test_forward_gather_last_step(B, nvec, L, dtype, device):
+    from modelos_amd import embedding_bag as eb
+
+    D = nvec * (4 if dtype == torch.float32 else 8)
+    B = B if L < 100 else min(B, 300)
+    W, idx, p, _ = eb_inputs(B, L, 300, D, dtype, seed=B + L, with_grad=False)
+    idx = idx.clamp_min(1)
+    W[0] = 0
+    expect = ref.eb_forward(idx, W, p)
+    cond = ref.eb_forward(idx, W.abs(), p.abs())
+    W[0] = float("inf")
+    out = eb.eb_forward(*_dev(idx, W, p, device=device))
+    assert_rel_close(out, expect, REL_TOL[dtype], f"forward {dtype} {B,L,D}", cond=cond)
+
+
 def test_forward_empty(device):
     from modelos_amd import embedding_bag as eb
 
