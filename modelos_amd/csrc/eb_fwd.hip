@@ -402,6 +402,10 @@ static void launch_fwd(const void* W, int64_t K, int64_t D, const int64_t* idx, 
 constexpr int64_t kGatherSliceBags = 8192;  // two bags a wave: half the chip's wave slots from one slice
 constexpr int64_t kGatherFill = 2048;       // waves under which a task's lookups are shared (8 a CU)
 
+// Waves of one launch: half the 2^32 threads that a grid can hold. Slices make
+// several waves of a wide row, so more bags than that go in several launches.
+constexpr int64_t kGatherMaxWaves = (int64_t)1 << 25;
+
 template <typename TW, int BPW>
 static void launch_gather(const void* W, int64_t K, int64_t D, const int64_t* idx, const void* psw, int pdt, int64_t B,
                           int64_t L, void* out, hipStream_t stream) {
@@ -411,10 +415,16 @@ static void launch_gather(const void* W, int64_t K, int64_t D, const int64_t* id
   int nw = 1;
   while (nw < kGatherMaxNW && tasks * nw < kGatherFill && L > (int64_t)kGatherLanes * nw) nw *= 2;
   const int waves = nw > 4 ? nw : 4;
+  const int64_t step = kGatherMaxWaves / S * BPW;  // bags per launch
   KernelSpan span("eb_fwd", stream);
-  hipLaunchKernelGGL((eb_gather_kernel<TW, BPW>), dim3((unsigned)((tasks * nw + waves - 1) / waves)), dim3(64 * waves),
-                     nw > 1 ? (size_t)waves * 64 * EPV * sizeof(float) : 0, stream, (const TW*)W, K, D, idx, psw, pdt,
-                     B, L, S, nw, (TW*)out);
+  for (int64_t b0 = 0; b0 < B; b0 += step) {
+    const int64_t nb = B - b0 < step ? B - b0 : step;
+    const int64_t n = (nb + BPW - 1) / BPW * S * nw;
+    const char* p = psw != nullptr ? (const char*)psw + (size_t)(b0 * L) * (size_t)elem_size(pdt) : nullptr;
+    hipLaunchKernelGGL((eb_gather_kernel<TW, BPW>), dim3((unsigned)((n + waves - 1) / waves)), dim3(64 * waves),
+                       nw > 1 ? (size_t)waves * 64 * EPV * sizeof(float) : 0, stream, (const TW*)W, K, D,
+                       idx != nullptr ? idx + b0 * L : nullptr, (const void*)p, pdt, nb, L, S, nw, (TW*)out + b0 * D);
+  }
 }
 
 // Rows of whole 16-vector pieces, and row numbers that fit a register (a
@@ -425,6 +435,7 @@ static bool try_gather(const void* W, int64_t K, int64_t D, const int64_t* idx, 
   constexpr int EPV = VecTraits<TW>::EPV;
   if (D % (kGatherLanes * EPV) != 0 || K >= 0xFFFFFFFFll) return false;
   const int64_t nvec = D / EPV;
+  if (nvec / 16 > kGatherMaxWaves) return false;
   if (nvec % 64 == 0 && B < kGatherSliceBags)
     launch_gather<TW, 1>(W, K, D, idx, psw, pdt, B, L, out, stream);
   else if (nvec % 32 == 0)

@@ -126,6 +126,28 @@ def test_forward_gather_last_step(B, nvec, L, dtype, device):
     assert_rel_close(out, expect, REL_TOL[dtype], f"forward {dtype} {B,L,D}", cond=cond)
 
 
+# More bags than one grid holds: two bags a wave, 16 slices of an 8 KB row, so
+# 2^23 bags are 2^26 waves (two launches; 64 GiB of output). One lookup a bag and
+# weights that are powers of two: the rows are exact.
+def test_forward_more_bags_than_a_grid(device):
+    from modelos_amd import embedding_bag as eb
+
+    B, K, D = (1 << 23) + 3, 257, 4096
+    if torch.cuda.mem_get_info(device)[0] < 100 << 30:
+        pytest.skip("needs 100 GiB of device memory")
+    gen = torch.Generator(device=device).manual_seed(5)
+    W = torch.randn((K, D), generator=gen, device=device).to(torch.bfloat16)
+    idx = torch.randint(0, K, (B, 1), generator=gen, device=device)
+    p = torch.tensor([0.5, 1.0, 2.0], device=device)[torch.randint(0, 3, (B, 1), generator=gen, device=device)]
+    out = eb.eb_forward(idx, W, p)
+    for a in range(0, B, 1 << 20):
+        rows = W[idx[a:a + (1 << 20), 0]]
+        rows *= p[a:a + (1 << 20)].to(torch.bfloat16)
+        assert torch.equal(out[a:a + (1 << 20)], rows), f"bags from {a}"
+    del out, rows
+    torch.cuda.empty_cache()
+
+
 def test_forward_empty(device):
     from modelos_amd import embedding_bag as eb
 
