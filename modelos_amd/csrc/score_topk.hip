@@ -1001,10 +1001,13 @@ __global__ __launch_bounds__(kThreads) void pkm_score_topk_kernel(
 #pragma unroll
       for (int i = 0; i < (64 + LPR - 1) / LPR; ++i) {
         const int j = sub + LPR * i;
-        if (j < knn) l0[j] = park[i];
+        if (j < knn) {
+          l0[j] = park[i];
+          if (!live) list[j] = (Key)0;  // (rows past the last token selected nothing)
+        }
       }
-      __builtin_amdgcn_wave_barrier();  // the first half's list of a row is written and read by its own lanes
-      cartesian_rows<TIN, LPR, MAXM, MAXS>(l0, list, cand, fin, L.cap, knn, sub, true, wscr, [&](int rr) {
+      __builtin_amdgcn_wave_barrier();  // the lists of a row are written and read by its own lanes
+      cartesian_rows<TIN, LPR, MAXM, MAXS>(l0, list, cand, fin, L.cap, knn, sub, live, wscr, [&](int rr) {
         const int row = w * RPW + rr;
         return CartRow<Key>{(const Key*)smem + row * L.kl, (const Key*)(R + L.list_off) + row * L.kl,
                             (Key*)smem + (TM + row) * L.kl};
