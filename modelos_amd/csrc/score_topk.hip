@@ -1765,9 +1765,14 @@ namespace pkm {
 // against 64). The selection's threshold needs groups enough for knn of their
 // maxima to be a tight bound: with fewer than 2 knn groups most rows take the
 // exact search and the streaming kernel is the faster one (256 keys, knn 32,
-// 512 tokens: 38 against 47).
-static int few_tokens_tile(int64_t tokens, int H, int n, int knn, int dtype, int max_tile) {
+// 512 tokens: 38 against 47). Where the streaming kernel takes the call
+// (`streams`), tiles of more than n / 8 tokens leave it too few keys to be ahead
+// of it: 128 keys, knn 8, 16 heads x 512 tokens 25.3 against 32.5 by tiles of 64;
+// 256 keys, knn 16, 3 heads x 2048 tokens of half 128 31.3 against 33.5, x 1001
+// by tiles of 32 31.2 against 26.4.
+static int few_tokens_tile(int64_t tokens, int H, int n, int knn, int dtype, bool streams, int max_tile) {
   if (dtype == PKM_DTYPE_BF16 && n < 16 * knn) return 0;
+  if (streams && max_tile > n / 8) max_tile = n / 8;
   const int64_t per_tile = dtype == PKM_DTYPE_BF16 ? 2 * (int64_t)H : H;
   for (int tile = 16; tile <= max_tile; tile *= 2)
     if ((tokens + tile - 1) / tile * per_tile <= 256) return tile;
@@ -1818,9 +1823,10 @@ static int score_topk_impl(const void* query, const void* keys, int64_t num_toke
   int TM = 64;
   while (TM > 16 && (score_lds_layout(TM, n, hf, k, esz, key_bytes).total > lds_max || n > score_max_n(TM, esz)))
     TM /= 2;
-  const int few = few_tokens_tile(num_tokens, H, n, k, dtype, TM);
-  if (!few && dtype == PKM_DTYPE_BF16 && score_type == PKM_SCORE_DOT && knn <= stream::kNet &&
-      (half == 128 || half == 256) && (int)stream::lds_bytes((int)half) <= lds_max) {
+  const bool streams = dtype == PKM_DTYPE_BF16 && score_type == PKM_SCORE_DOT && knn <= stream::kNet &&
+                       (half == 128 || half == 256) && (int)stream::lds_bytes((int)half) <= lds_max;
+  const int few = few_tokens_tile(num_tokens, H, n, k, dtype, streams, TM);
+  if (!few && streams) {
     const int64_t blocks = ((num_tokens + stream::kTok - 1) / stream::kTok) * 2 * heads;
     PKM_REQUIRE(blocks < ((int64_t)1 << 31), PKM_ERR_INVALID_ARGUMENT, "pkm_score_topk: grid too large");
     const bool sub = out_sub_scores1 != nullptr || out_sub_scores2 != nullptr;

@@ -206,6 +206,22 @@ def test_few_and_many_tokens_agree(device, case, knn):
             assert torch.equal(a, b[: a.shape[0]]), f"{case} knn {knn} tokens {tokens}"
 
 
+# Few keys: tiles of at most n / 8 tokens, the streaming kernel past the tokens
+# that those hold (2 heads: 16-token tiles up to 1024 tokens of 128 keys,
+# 32-token ones up to 2048 of 256 keys).
+@pytest.mark.parametrize("n,knn,edge", [(64, 4, 1), (128, 8, 1024), (256, 16, 2048), (320, 16, 2048)])
+def test_few_tokens_few_keys_agree(device, n, knn, edge):
+    H, half = 2, 128
+    g = gen(400 + n)
+    q = torch.randn((89, H, 2 * half), generator=g).to(torch.bfloat16)
+    k = (torch.randn((2 * H * n, half), generator=g) * half**-0.5).to(torch.bfloat16)
+    many = _run(_repeat_tokens(q, 4353), k, H, knn, device)
+    for tokens in (1, edge, edge + 1, 4096):
+        few = _run(_repeat_tokens(q, tokens), k, H, knn, device)
+        for a, b in zip(few, many):
+            assert torch.equal(a, b[: a.shape[0]]), f"tokens {tokens}"
+
+
 # The rule's other routes: more lanes per row in the cartesian step up to 8192
 # rows, smaller tiles of float32 and of key dims the streaming kernel does not
 # take, dead rows of a tile (their equal scores select nothing).
