@@ -1596,11 +1596,14 @@ __host__ inline size_t lds_bytes(int half) {
 
 // Lanes per row of the cartesian kernel: 8 in bulk, 16 for knn > 32 (280 pairs a
 // row at knn 64: scoring + cartesian of 65536 rows 573 -> 545 us; knn 32, 131072
-// rows, 287 -> 304); 32 up to 8192 rows, where
-// the row's serial chain is what it takes (knn 32, up to 4096 rows: scoring +
-// cartesian 2 to 4 us less; knn 64, 4096 rows 75 -> 63 us, 8192 rows 102 ->
-// 95; 16384 rows of knn 32 72 -> 80).
-constexpr int64_t kCartWideRows = 8192;
+// rows, 287 -> 304); 32 for few rows, where the row's serial chain is what it
+// takes: up to 4096 rows (knn 32, 4096 rows of 512 keys: scoring + cartesian 35.6
+// us by 8 lanes, 32.8 by 32; knn 8, 5000 rows of 128 keys 25.1 and 26.6), and to
+// 8192 for knn > 32 (knn 64, 4096 rows 75 -> 63 us, 8192 rows 102 -> 95).
+static int cartesian_lanes(int64_t rows, int knn) {
+  if (knn > 32) return rows <= 8192 ? 32 : 16;
+  return rows <= 4096 ? 32 : 8;
+}
 __host__ inline size_t cartesian_lds_bytes(int knn, int lpr) {
   const int kl = (knn + 3) & ~3;
   return (size_t)(kThreads / lpr) * (size_t)(3 * kl + score_cap(knn, lpr) + 4) * 4;
@@ -1646,9 +1649,14 @@ template <typename TIN>
 static int launch_cartesian(int64_t Ntok, int H, int n, int knn, int lds_max, void* out_scores, int64_t* out_idx,
                             hipStream_t st) {
   const int64_t rows = Ntok * H;
-  if (rows <= kCartWideRows) return launch_cartesian_lpr<TIN, 32>(rows, n, knn, lds_max, out_scores, out_idx, st);
-  return knn > 32 ? launch_cartesian_lpr<TIN, 16>(rows, n, knn, lds_max, out_scores, out_idx, st)
-                  : launch_cartesian_lpr<TIN, 8>(rows, n, knn, lds_max, out_scores, out_idx, st);
+  switch (cartesian_lanes(rows, knn)) {
+    case 32:
+      return launch_cartesian_lpr<TIN, 32>(rows, n, knn, lds_max, out_scores, out_idx, st);
+    case 16:
+      return launch_cartesian_lpr<TIN, 16>(rows, n, knn, lds_max, out_scores, out_idx, st);
+    default:
+      return launch_cartesian_lpr<TIN, 8>(rows, n, knn, lds_max, out_scores, out_idx, st);
+  }
 }
 
 template <typename TIN, int IDW, int TM, int KSC>
