@@ -1762,8 +1762,8 @@ __global__ __launch_bounds__(256) void score_keys_pack_kernel(const uint4* __res
 
 namespace pkm {
 // Tokens per tile of the tile kernel where the tokens are too few to fill the
-// chip: the smallest tile whose workgroups fit it in one round (bf16: one half
-// each), 0 where not even the largest tile's do. The scores are the same bits
+// chip: the smallest tile whose workgroups fit its `cus` CUs in one round (bf16:
+// one half each), 0 where not even the largest tile's do. The scores are the same bits
 // as the streaming kernel's (both sum a dot product in ascending k-steps of
 // the matrix cores), which takes a whole workgroup and the same time for 1 to
 // 256 tokens of a (head, half). Scoring + cartesian step, bf16, knn 32, half
@@ -1778,12 +1778,12 @@ namespace pkm {
 // of it: 128 keys, knn 8, 16 heads x 512 tokens 25.3 against 32.5 by tiles of 64;
 // 256 keys, knn 16, 3 heads x 2048 tokens of half 128 31.3 against 33.5, x 1001
 // by tiles of 32 31.2 against 26.4.
-static int few_tokens_tile(int64_t tokens, int H, int n, int knn, int dtype, bool streams, int max_tile) {
+static int few_tokens_tile(int64_t tokens, int H, int n, int knn, int dtype, bool streams, int max_tile, int cus) {
   if (dtype == PKM_DTYPE_BF16 && n < 16 * knn) return 0;
   if (streams && max_tile > n / 8) max_tile = n / 8;
   const int64_t per_tile = dtype == PKM_DTYPE_BF16 ? 2 * (int64_t)H : H;
   for (int tile = 16; tile <= max_tile; tile *= 2)
-    if ((tokens + tile - 1) / tile * per_tile <= 256) return tile;
+    if ((tokens + tile - 1) / tile * per_tile <= cus) return tile;
   return 0;
 }
 }  // namespace pkm
@@ -1808,9 +1808,10 @@ static int score_topk_impl(const void* query, const void* keys, int64_t num_toke
               PKM_ERR_INVALID_ARGUMENT, "pkm_score_topk: score outputs must be 4-byte aligned");
   const int esz = dtype == PKM_DTYPE_BF16 ? 2 : 4;  // score-tile element = order key of the input dtype
   const int key_bytes = dtype == PKM_DTYPE_BF16 ? 4 : 8;
-  int dev = 0, lds_max = 0;
+  int dev = 0, lds_max = 0, cus = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (e != hipSuccess)
     return pkm_set_error(PKM_ERR_HIP, "pkm_score_topk: device query failed: %s", hipGetErrorString(e));
   if (lds_max > kMaxLds) lds_max = kMaxLds;
@@ -1833,7 +1834,7 @@ static int score_topk_impl(const void* query, const void* keys, int64_t num_toke
     TM /= 2;
   const bool streams = dtype == PKM_DTYPE_BF16 && score_type == PKM_SCORE_DOT && knn <= stream::kNet &&
                        (half == 128 || half == 256) && (int)stream::lds_bytes((int)half) <= lds_max;
-  const int few = few_tokens_tile(num_tokens, H, n, k, dtype, streams, TM);
+  const int few = few_tokens_tile(num_tokens, H, n, k, dtype, streams, TM, cus);
   if (!few && streams) {
     const int64_t blocks = ((num_tokens + stream::kTok - 1) / stream::kTok) * 2 * heads;
     PKM_REQUIRE(blocks < ((int64_t)1 << 31), PKM_ERR_INVALID_ARGUMENT, "pkm_score_topk: grid too large");
