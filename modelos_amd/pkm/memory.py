@@ -131,20 +131,33 @@ def _column_sum(g: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.
 _PLAIN_TENSORS = (torch.Tensor, nn.Parameter)
 
 
+def _rows_kernel_sizes(rows: int, inputs: int, outputs: int) -> bool:
+    """Whether pkm_linear_rows takes these sizes and is the faster one at
+    them: its time grows with the inputs and, past 16 rows, with the rows; the
+    BLAS's hardly below 64 rows. In us, BLAS / pkm_linear_rows, inputs x
+    outputs: 1024 x 1024, 8 rows 5.3 / 3.4, 64 rows 7.5 / 6.8; 1056 x 1024, 64
+    rows 6.2 / 5.3; 1536 x 1024, 16 rows 5.9 / 5.5, 64 rows 5.9 / 11.2; 4096 x
+    4096, 16 rows 13.0 / 9.9, 17 rows 10.8 / 12.2; 6144 x 1024, 8 rows 8.4 /
+    10.9; and past one workgroup of 16 outputs per CU, 2048 x 16384, 8 rows
+    14.6 / 16.1, 64 rows 15.9 / 42.9."""
+    return (0 < rows <= 64 and inputs % 32 == 0 and outputs % 16 == 0
+            and 0 < inputs <= (4096 if rows <= 16 else 1056) and 0 < outputs <= 4096)
+
+
 def _rows_kernel_takes(x, weight, bias) -> bool:
-    """Whether pkm_linear_rows serves these operands: up to 64 bf16 rows of
-    plain, contiguous, aligned tensors on one GPU (above, the BLAS's tiles
-    are full: 64 rows of 1024 x 1024 take 5 us here and 7 us there)."""
-    if x.dim() != 2 or not 0 < x.shape[0] <= 64 or x.dtype != torch.bfloat16 or not x.is_cuda:
+    """Whether pkm_linear_rows serves these operands: few bf16 rows of plain,
+    contiguous, aligned tensors on one GPU."""
+    if x.dim() != 2 or weight.dim() != 2 or x.dtype != torch.bfloat16 or not x.is_cuda:
         return False
     if type(x) not in _PLAIN_TENSORS or type(weight) not in _PLAIN_TENSORS or x.shape[1] != weight.shape[1]:
         return False
+    if not _rows_kernel_sizes(x.shape[0], x.shape[1], weight.shape[0]):
+        return False
     if bias is not None and (type(bias) not in _PLAIN_TENSORS or bias.dtype != x.dtype or bias.device != x.device
-                             or not bias.is_contiguous()):
+                             or bias.shape != weight.shape[:1] or not bias.is_contiguous()):
         return False
     return (weight.dtype == x.dtype and weight.device == x.device and x.is_contiguous() and weight.is_contiguous()
-            and x.shape[1] % 32 == 0 and weight.shape[0] % 16 == 0 and x.data_ptr() % 16 == 0
-            and weight.data_ptr() % 16 == 0)
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
 def _linear(layer: nn.Linear, x: torch.Tensor, few_rows: bool = False) -> torch.Tensor:

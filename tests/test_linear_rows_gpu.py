@@ -30,14 +30,19 @@ def test_against_float64(device, rows, fin, fout, bias):
             lin.bias.copy_(torch.randn(fout, generator=g))
     lin = lin.to(device=device, dtype=torch.bfloat16)
     x = torch.randn((rows, fin), generator=g).to(torch.bfloat16).to(device)
-    assert memory._rows_kernel_takes(x, lin.weight, lin.bias)
-    y = memory._linear(lin, x, True)
+    # (at the last size the layer calls the BLAS, which is the faster one there)
+    takes = memory._rows_kernel_takes(x, lin.weight, lin.bias)
+    assert takes == (rows <= 16 or fin <= 1056)
+    y = torch.empty((rows, fout), dtype=torch.bfloat16, device=device)
+    _lib.call("pkm_linear_rows", _lib.ptr(x), _lib.ptr(lin.weight), _lib.ptr(lin.bias), rows, fin, fout,
+              _lib.dtype_code(x), _lib.ptr(y), _lib.stream_of(x.device))
     w64, x64 = lin.weight.detach().double(), x.double()
     b64 = lin.bias.detach().double() if bias else torch.zeros(fout, dtype=torch.float64, device=device)
     expect = x64 @ w64.t() + b64
     bound = (x64.abs() @ w64.abs().t() + b64.abs()) * 2.0**-20 + expect.abs() * 2.0**-8
     assert ((y.double() - expect).abs() <= bound).all()
-    assert torch.equal(y, memory._linear(lin, x, True))
+    if takes:
+        assert torch.equal(y, memory._linear(lin, x, True))
 
 
 def test_what_it_does_not_take(device):
@@ -48,8 +53,21 @@ def test_what_it_does_not_take(device):
     assert not memory._rows_kernel_takes(x[:8, ::2], lin.weight[:, :32], lin.bias)  # strides
     assert not memory._rows_kernel_takes(x[:8].float(), lin.weight.float(), lin.bias.float())
     assert not memory._rows_kernel_takes(x.reshape(-1)[1:8 * 64 + 1].view(8, 64), lin.weight, lin.bias)  # alignment
+    assert not memory._rows_kernel_takes(x[:8], lin.weight, lin.bias[:1])  # a bias that broadcasts
     y = torch.empty((8, 32), dtype=torch.bfloat16, device=device)
     for rows, fin, fout, code in ((65, 64, 32, 1), (8, 48, 32, 1), (8, 64, 24, 1), (8, 64, 32, 0)):
         with pytest.raises(_lib.PkmError):
             _lib.call("pkm_linear_rows", _lib.ptr(x), _lib.ptr(lin.weight), None, rows, fin, fout, code, _lib.ptr(y),
                       _lib.stream_of(x.device))
+
+
+# Sizes that the kernel does not take, or is the slower one at, go to F.linear.
+def test_sizes_past_the_rule_run(device):
+    for rows, fin, fout in ((3, 0, 16), (3, 32, 0), (17, 1088, 16), (16, 4128, 16), (2, 1 << 20, 16), (2, 64, 4112)):
+        lin = torch.nn.Linear(fin, fout).to(device=device, dtype=torch.bfloat16) if fin and fout else None
+        w = lin.weight if lin else torch.zeros((fout, fin), dtype=torch.bfloat16, device=device)
+        b = lin.bias if lin else torch.ones(fout, dtype=torch.bfloat16, device=device)
+        x = torch.randn((rows, fin), device=device).to(torch.bfloat16)
+        assert not memory._rows_kernel_takes(x, w, b)
+        y = memory._Linear.apply(x, w, b, True)
+        assert torch.equal(y, torch.nn.functional.linear(x, w, b))

@@ -7,7 +7,7 @@ import pytest
 import torch
 from torch import nn
 
-from modelos_amd.pkm.memory import _linear, _weight_grad_splits
+from modelos_amd.pkm.memory import _linear, _rows_kernel_sizes, _weight_grad_splits
 from tests.helpers import REL_TOL, assert_rel_close, gen
 
 
@@ -36,6 +36,15 @@ def test_split_heuristic():
     assert _weight_grad_splits(4096, 1024, 1024) == 2
     assert _weight_grad_splits(3000, 1024, 1024) == 1  # below 2 x 2048 rows
     assert _weight_grad_splits(16384 + 2, 1024, 1024) == 2  # rows must divide evenly
+
+
+def test_rows_kernel_sizes():
+    for rows, inputs, outputs in ((1, 32, 16), (16, 4096, 4096), (17, 1056, 1024), (64, 1024, 4096)):
+        assert _rows_kernel_sizes(rows, inputs, outputs)
+    # no rows, inputs or outputs; past the kernel's own limits; slower than the BLAS
+    for rows, inputs, outputs in ((0, 32, 16), (1, 0, 16), (1, 32, 0), (65, 32, 16), (1, 48, 16), (1, 32, 24),
+                                  (1, 1 << 20, 16), (17, 1088, 16), (16, 4128, 16), (64, 4096, 64), (8, 2048, 16384)):
+        assert not _rows_kernel_sizes(rows, inputs, outputs)
 
 
 @pytest.mark.gpu
