@@ -1455,7 +1455,10 @@ __device__ __forceinline__ int hot_slot(uint32_t r, bool valid, const uint32_t* 
 
 // Chunk pointers, chunk-major (index c * hr_max + i): pc and po of (chunk c,
 // list position i) = the first sorted occurrence of the row hot[i] in a bag >=
-// 32 c, for c = 0..nc (c = nc: the row's end). hot_entries_kernel flags pc.
+// 32 c, for c = 0..nc (c = nc: the row's end). hot_entries_kernel flags pc. A
+// long run of chunks without the row (after its last bag, say) is written by the
+// wave, not by the one lane that finds it (2^20 bags x 8 into 2^17 x 512, 16 rows
+// that are hot in a sixteenth of the bags each: backward 13.34 -> 13.05 ms).
 __global__ __launch_bounds__(256) void hot_chunks_kernel(const uint32_t* __restrict__ hot, int64_t hr_max,
                                                          const uint32_t* __restrict__ offs,
                                                          const uint32_t* __restrict__ skeys,
@@ -1471,18 +1474,35 @@ __global__ __launch_bounds__(256) void hot_chunks_kernel(const uint32_t* __restr
     const bool valid = j < nv;
     uint32_t beg = 0, end = 0;
     const int i = hot_slot(valid ? skeys[j] : 0u, valid, hot, n, offs, hot_min, &beg, &end);
-    if (i < 0) continue;
-    // chunks (chunk of the row's previous occurrence, chunk of this one] start here
-    const uint32_t c = meta[j].x / kHotKC;
-    for (uint32_t cc = j == beg ? 0u : meta[j - 1].x / kHotKC + 1u; cc <= c; ++cc) {
-      pc[cc * H + i] = j;
-      po[cc * H + i] = j;
+    // chunks [c0, c1), after the row's previous occurrence's up to this one's, start at j; past the last
+    // occurrence's, [c1, c2) at the row's end
+    uint32_t c0 = 0, c1 = 0, c2 = 0;
+    if (i >= 0) {
+      c0 = j == beg ? 0u : meta[j - 1].x / kHotKC + 1u;
+      c1 = meta[j].x / kHotKC + 1u;
+      c2 = j + 1 == end ? nc + 1 : c1;
     }
-    if (j + 1 == end)
-      for (uint32_t cc = c + 1; cc <= nc; ++cc) {
-        pc[cc * H + i] = end;
-        po[cc * H + i] = end;
+    auto put = [&](uint32_t from, uint32_t to, uint32_t v) {
+      const bool far = to - from > 8u;  // by the wave
+      if (!far)
+        for (uint32_t cc = from; cc < to; ++cc) {
+          pc[cc * H + i] = v;
+          po[cc * H + i] = v;
+        }
+      for (uint64_t m = __ballot(far); m != 0; m &= m - 1) {
+        const int l = __builtin_ctzll(m);
+        const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)from, l);
+        const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)to, l);
+        const uint32_t w = (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+        const uint32_t slot = (uint32_t)__builtin_amdgcn_readlane(i, l);
+        for (uint32_t cc = f + (threadIdx.x & 63); cc < t; cc += 64) {
+          pc[cc * H + slot] = w;
+          po[cc * H + slot] = w;
+        }
       }
+    };
+    put(c0, c1, j);
+    put(c1, c2, end);
   }
 }
 

@@ -638,6 +638,35 @@ def test_backward_hot_rows_chunk_densities(L, device):
     assert torch.equal(gW, gW2) and torch.equal(gp, gp2)
 
 
+# Hot rows with long runs of 32-bag chunks that do not hold them (written by a
+# wave, shorter ones by a lane: 8 chunks and 9): before the first, between two,
+# after the last; the end of one such row and the start of the next in one wave.
+def test_backward_hot_rows_chunk_gaps(device):
+    from modelos_amd import embedding_bag as eb
+
+    B, L, K, D = 4100, 6, 3000, 512
+    W, _, p, g = eb_inputs(B, L, K, D, torch.bfloat16, seed=91)
+    idx = torch.randint(100, K, (B, L), generator=torch.Generator().manual_seed(92))
+    idx[600:900, 0] = 5  # then 100 chunks without
+    idx[-300:, 0] = 6
+    idx[1000:1200, 0] = 7  # before, between and after
+    idx[3000:3100, 0] = 7
+    for c in range(0, B - 64, 9 * 32):  # every ninth chunk
+        idx[c:c + 32, 1] = 8
+    for c in range(0, B - 64, 10 * 32):
+        idx[c:c + 32, 2] = 9
+    for r in range(8):  # rows 10 to 17: 260 lookups each, 44 bags
+        idx[64 * r:64 * r + 44] = 10 + r
+        idx[64 * r + 43, 4:] = 20
+    gW, gp = eb.eb_backward(*_dev(idx, W, p, g, device=device))
+    eW, ep = ref.eb_backward(idx, W, p, g)
+    cW, cp = ref.eb_backward(idx, W.abs(), p.abs(), g.abs())
+    assert_rel_close(gW, eW, REL_TOL[torch.bfloat16], "grad_weight", cond=cW)
+    assert_rel_close(gp, ep, REL_TOL[torch.bfloat16], "grad_psw", cond=cp)
+    gW2, gp2 = eb.eb_backward(*_dev(idx, W, p, g, device=device))
+    assert torch.equal(gW, gW2) and torch.equal(gp, gp2)
+
+
 # The sparse plan's edges: the one-workgroup sort's last size and the two-level
 # sort after it, the last row count it takes and one row fewer (the general
 # plan), one and two keys of 8-bit digits; runs of 1 to 300 lookups across
