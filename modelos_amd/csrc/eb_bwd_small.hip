@@ -283,10 +283,14 @@ __global__ __launch_bounds__(256) void sparse_narrow_kernel(const TW* __restrict
 // The out-of-range lookups' psw-gradients are zeroed on the way: the sorted
 // ones past nvalid (small_sort), or the list `invalid`.
 // (A wave per lookup pays five dependent reads for each: backward of 262144
-// lookups into 2^20 x 1024 bf16 803 us, 624 so.) Windows of 16 lookups, of 4
-// where there are too few of those to fill the chip.
+// lookups into 2^20 x 1024 bf16 803 us, 624 so.) Windows of 16 lookups, of 4 up to
+// kWinFewLookups, where there are too few of the others to fill the chip: 2^20 x
+// 1024 bf16, windows of 4 / 16, 4096 lookups 25.7 / 32.0 us, 10240 50.5 / 55.5,
+// 65536 154 / 158 (Zipf(1.1) 214 / 204), 262144 374 / 374 (334 / 309); 2^19 x 2048
+// f32, 100000 538 / 568 (451 / 436).
 constexpr int kWin = 16;
 constexpr int kWinFew = 4;
+constexpr int64_t kWinFewLookups = 163840;
 
 template <typename TW, typename TG, int VPL, bool ACC>
 __global__ __launch_bounds__(256) void sparse_runs_kernel(const TW* __restrict__ W, int64_t D,
@@ -479,7 +483,7 @@ static void launch_sparse(const void* W, int64_t K, int64_t D, const void* psw, 
   const int64_t nchunks = N > kHeavyT ? (N + kHeavyT - 1) / kHeavyT : 0;
   KernelSpan span("eb_bwd_rows", st);
   if constexpr (LPG == 64) {
-    const int win = N > 16 * kSmallLookups ? kWin : kWinFew;
+    const int win = N > kWinFewLookups ? kWin : kWinFew;
     const int64_t waves = (N + win - 1) / win + nchunks;
     hipLaunchKernelGGL((sparse_runs_kernel<TW, TG, VPL, ACC>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st,
                        (const TW*)W, D, psw, pdt, (const TG*)g, (uint32_t)L, skeys, svals, nvalid, (uint32_t)N,
