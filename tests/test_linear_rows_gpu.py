@@ -71,3 +71,27 @@ def test_sizes_past_the_rule_run(device):
         assert not memory._rows_kernel_takes(x, w, b)
         y = memory._Linear.apply(x, w, b, True)
         assert torch.equal(y, torch.nn.functional.linear(x, w, b))
+
+
+def test_infinities_and_nan(device):
+    """An infinite or NaN row of x reaches its own row of y only, one of the
+    weight its own column; rows past the last tile's are copies of the last."""
+    rows, fin, fout = 9, 96, 32
+    g = gen(77)
+    x = torch.randn((rows, fin), generator=g).to(torch.bfloat16)
+    w = torch.randn((fout, fin), generator=g).to(torch.bfloat16)
+    x[2, 5], x[8, 95], w[17, 40] = float("inf"), float("nan"), float("-inf")
+    lin = torch.nn.Linear(fin, fout)
+    with torch.no_grad():
+        lin.weight.copy_(w.float())
+    lin = lin.to(device=device, dtype=torch.bfloat16)
+    x = x.to(device)
+    assert memory._rows_kernel_takes(x, lin.weight, lin.bias)
+    y = memory._linear(lin, x, True).double()
+    expect = x.double() @ lin.weight.detach().double().t() + lin.bias.detach().double()
+    assert torch.equal(y.isnan(), expect.isnan())
+    inf = expect.isinf()
+    assert torch.equal(y[inf], expect[inf])
+    fine = expect.isfinite()
+    bound = expect.abs() * 2.0**-8 + fin * 2.0**-18
+    assert ((y - expect).abs()[fine] <= bound[fine]).all()

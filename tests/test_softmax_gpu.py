@@ -78,3 +78,24 @@ def test_long_rows_extreme_scores(device):
     torch.cuda.synchronize()
     assert_rel_close(y, e_y, 1e-6, "y")
     assert_rel_close(dx, e_dx, 1e-5, "dx")
+
+
+# dx = p (dy - <dy, p>) cancels where a row is close to one-hot: compared with
+# float64 relative to the size of its terms, p (|dy| + <|dy|, p>). Bounds: one
+# rounding of a 16-bit output (2^-8, 2^-11) and 64 float32 roundings (exp of a
+# rounded difference, the sums over a row) of 2^-24 relative to the terms.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16], ids=["bf16", "f32", "f16"])
+@pytest.mark.parametrize("shape", [(2, 24), (50, 24), (99, 16), (40, 128), (33, 65), (21, 256)], ids=str)
+def test_gradient_relative_to_its_terms(device, dtype, shape):
+    g = gen(15)
+    x = (torch.randn(shape, generator=g) * 4).to(dtype).to(device)
+    dy = torch.randn(shape, generator=g).to(dtype).to(device)
+    y, dx = _run(score_softmax, x, dy)
+    p = torch.softmax(x.double(), -1)
+    d = dy.double()
+    expect = p * (d - (d * p).sum(-1, keepdim=True))
+    terms = p * (d.abs() + (d.abs() * p).sum(-1, keepdim=True))
+    eps = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11, torch.float32: 0.0}[dtype] + 64 * 2.0**-24
+    floor = 2.0**-24 if dtype == torch.float16 else 0.0  # its smallest subnormal
+    assert ((dx.double() - expect).abs() <= eps * terms + floor).all()
+    assert ((y.double() - p).abs() <= eps * p + floor).all()
