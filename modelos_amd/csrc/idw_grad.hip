@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void row_sumsq_kernel(const float* __restrict_
 
 static int idw_check(const char* what, int64_t batches, int64_t rows, int64_t dim) {
   PKM_REQUIRE(batches >= 0 && rows >= 0 && dim > 0, PKM_ERR_INVALID_ARGUMENT, "%s: bad sizes", what);
-  PKM_REQUIRE(dim % 4 == 0 && dim < ((int64_t)1 << 20) && batches * rows < ((int64_t)1 << 35), PKM_ERR_UNSUPPORTED,
+  PKM_REQUIRE(dim % 4 == 0 && dim < ((int64_t)1 << 30) && batches * rows < ((int64_t)1 << 35), PKM_ERR_UNSUPPORTED,
               "%s: %lld x %lld rows of %lld not supported (rows of whole 16-byte vectors)", what, (long long)batches,
               (long long)rows, (long long)dim);
   return PKM_OK;

@@ -222,9 +222,10 @@ def _idw_grad_coef(dS, qq, kk, dots):
 
 
 def _vector_rows(*tensors) -> bool:
-    """Contiguous float32 tensors of 16-byte aligned rows of whole vectors."""
+    """Contiguous float32 tensors of 16-byte aligned rows of whole vectors, of
+    the lengths that the row kernels take."""
     return all(t.dtype == torch.float32 and t.is_contiguous() and t.shape[-1] % 4 == 0 and t.data_ptr() % 16 == 0
-               for t in tensors)
+               and 0 < t.shape[-1] < 1 << 30 for t in tensors)
 
 
 def _row_sumsq(x, row_major):

@@ -35,3 +35,17 @@ def test_finish_and_sumsq(device, B, T, dim, row_major):
         o = pk._idw_finish(R, y, s, row_major)
         yb = y.transpose(0, 1) if row_major else y
         assert torch.equal(o.transpose(0, 1) if row_major else o, 2.0 * (R - yb * s[:, :, None]))
+
+
+def test_long_and_empty_rows(device):
+    """Rows of 4 MB are the kernels' too; rows of no length are zeros."""
+    B, T, dim = 2, 3, 1 << 20
+    P = torch.randn((B, T, dim), device=device)
+    x = torch.randn((T, B, dim), device=device)
+    s = torch.randn((B, T), device=device)
+    out = pk._idw_finish(P, x, s, True)
+    assert torch.equal(out.transpose(0, 1), 2.0 * (P - x.transpose(0, 1) * s[:, :, None]))
+    q = pk._row_sumsq(x, True)
+    e = x.transpose(0, 1).double().square().sum(-1)
+    assert ((q.double() - e).abs() <= e * dim / 16 * 2.0**-24).all()  # 16 chains a row
+    assert torch.equal(pk._row_sumsq(x[..., :0].contiguous(), True), torch.zeros((B, T), device=device))
