@@ -50,8 +50,9 @@ const char* pkm_last_error_string(void);
 /*
  * Weighted embedding bag, forward (mode "sum").
  *   out[b, :] = sum_{j < bag_size} psw[b, j] * weight[indices[b, j], :]
- * Accumulates in float32 in j order (for bags too few to fill the GPU in up to
- * 16 partial sums, added in a fixed order) and rounds once to weight's dtype.
+ * Accumulates in float32 in j order and rounds once to weight's dtype. For bags
+ * too few to fill the GPU the sum runs in up to 16 partial sums, added in a fixed
+ * order: the last float32 bits of a bag depend on how many bags the call has.
  * psw may be NULL (psw_dtype PKM_DTYPE_NONE): all weights are 1.
  * out: [bags, dim] in weight_dtype.
  *
@@ -80,10 +81,13 @@ size_t pkm_eb_bwd_workspace_size(int64_t num_rows, int64_t dim, int64_t bags, in
  * PKM_ERR_UNSUPPORTED (a caller widens a 16-bit gradient to float32 first,
  * which is exact).
  * workspace: device buffer of at least pkm_eb_bwd_workspace_size() bytes.
- * Rows with at least max(257, bags / 16) lookups (a BF16 table and grad_out,
- * dim a multiple of 512) are reduced as dense bf16 matrix products on the
+ * A row's float32 sums run over its lookups in position order; a row of more
+ * than 256 lookups in chunks of 256 sorted lookups, the chunks' sums added in order.
+ * Except: with more than max(10240, num_rows / 4) lookups, rows with at least
+ * max(257, bags / 16) of them (a BF16 table and grad_out, dim a multiple of 512,
+ * num_rows from 257 to 2^22) are reduced as dense bf16 matrix products on the
  * matrix cores, their weights merged per bag: float32 sums in a fixed order
- * (deterministic), not in position order as the other rows' are.
+ * (deterministic), not in position order.
  *
  * Replaces embedding_bag_bw_rev_indices
  *   (pkm/xformer_embeddingbag.py:331-386, fwpkm/xformer_embeddingbag_legacy.py:170-227),
@@ -101,10 +105,14 @@ int pkm_eb_bwd(const void* weight, int64_t num_rows, int64_t dim, int weight_dty
  * pkm_eb_bwd in two steps, so that the part that depends only on the lookups
  * can run early (e.g. during the forward pass, on another stream, beside the
  * gather) and the backward pass keeps only the reduction:
- *   pkm_eb_bwd_prepare  sorts the lookups by row, builds the row offsets, the
- *                       per-lookup metadata (bag, weight) and the row
- *                       kernel's lists in `workspace`. It reads indices and
- *                       psw, not weight or grad_out.
+ *   pkm_eb_bwd_prepare  sorts the lookups by row and builds in `workspace` what
+ *                       the reduction for these sizes reads beside them: the
+ *                       row offsets, the per-lookup metadata (bag, weight)
+ *                       and the row kernel's lists; or the sorted lookups
+ *                       alone, with at most 10240 lookups, or num_rows / 4
+ *                       (rows of 64 16-byte vectors or more, num_rows from
+ *                       257 to 2^22). It reads indices and psw, not weight
+ *                       or grad_out.
  *   pkm_eb_bwd_prepared runs the reduction (grad_weight, grad_psw) on a
  *                       workspace that pkm_eb_bwd_prepare filled, with the
  *                       same num_rows, dim, weight_dtype, indices, psw, bags
@@ -513,7 +521,7 @@ int pkm_swilu_bwd(const void* dh, const void* e, const void* s, int64_t n, int d
  * * row_factors[b, t]) over batches x rows rows of dim. products [batches, rows,
  * dim], row_factors [batches, rows]; x and out [rows, batches, dim] with
  * row_major (queries), else [batches, rows, dim] (keys). Every step rounded, no
- * contraction. dim a multiple of 4, buffers 16-byte aligned.
+ * contraction. dim a multiple of 4 below 2^30, buffers 16-byte aligned.
  *
  * Replaces part of the autograd of cdist (fwpkm/fwpkm.py:853-869).
  */
@@ -528,8 +536,10 @@ int pkm_row_sumsq(const float* x, int64_t batches, int64_t rows, int64_t dim, in
  * A Linear over a few rows: y[i, o] = bf16(sum_k x[i, k] * weight[o, k] + bias[o]),
  * float32 sums, one rounding. x [rows, in_features], weight [out_features,
  * in_features], bias [out_features] or NULL, y [rows, out_features]; bfloat16,
- * rows <= 64, in_features a multiple of 32, out_features of 16, x and weight
- * 16-byte aligned: PKM_ERR_UNSUPPORTED otherwise.
+ * rows <= 64, in_features a multiple of 32 below 2^20, out_features one of 16 below
+ * 2^24: PKM_ERR_UNSUPPORTED otherwise. x and weight 16-byte aligned:
+ * PKM_ERR_INVALID_ARGUMENT otherwise. Meant for few inputs: with many the
+ * BLAS's product is the faster one.
  *
  * Replaces F.linear of the value projections (pkm/memory.py:222-229) for the
  * few rows of a decode step.

@@ -6,9 +6,10 @@
 // waves owns 16 outputs; its waves split the inputs, each issuing its loads
 // (16-byte fragments of v_mfma_f32_16x16x32_bf16, straight from global memory)
 // before its first product; the float32 partial tiles meet in LDS, are summed
-// in wave order, get the bias and are rounded once. 8 rows, 1024 x 1024: 4 us
-// where the BLAS call took 6 us on the GPU and 27 us of host time a call; at
-// 64 rows 5 us against 7.
+// in wave order, get the bias and are rounded once. 8 rows, 1024 x 1024: 3.4 us
+// where the BLAS call took 5.3 us on the GPU and 27 us of host time a call; at
+// 64 rows 6.8 us against 7.5. With many inputs a wave's chain of products is too
+// long and the BLAS is ahead (the caller's rule: memory.py, _rows_kernel_sizes).
 #include "pkm_common.h"
 
 namespace pkm {

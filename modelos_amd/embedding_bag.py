@@ -69,7 +69,10 @@ def eb_forward(
 ) -> torch.Tensor:
     """out[b, :] = sum_j psw[b, j] * weight[indices[b, j], :], in weight.dtype.
 
-    float32 accumulation in j order (pkm/xformer_embeddingbag.py:97-113).
+    float32 accumulation in j order (pkm/xformer_embeddingbag.py:97-113); for
+    bags too few to fill the GPU in up to 16 partial sums, added in a fixed
+    order, so the last float32 bits of a bag depend on how many bags the call
+    has.
     """
     _check_bag_inputs(indices, weight, per_sample_weights, "eb_forward")
     dev = _require_device(indices, weight, per_sample_weights)
