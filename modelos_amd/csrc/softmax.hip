@@ -223,12 +223,13 @@ __global__ __launch_bounds__(256) void softmax_bwd_wave_kernel(const void* __res
   }
 }
 
-// lanes per row for the vector path (0: another path)
-static int sm_vec_lanes(int64_t cols, int dtype, const void* a, const void* b, const void* c) {
+// lanes per row for the vector path (0: another path; also where the lanes of all
+// rows are more than the 2^32 threads of a grid)
+static int sm_vec_lanes(int64_t rows, int64_t cols, int dtype, const void* a, const void* b, const void* c) {
   const int64_t bytes = cols * (dtype == PKM_DTYPE_BF16 ? 2 : 4);
   if ((((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) != 0) return 0;
-  if (bytes >= 16 && bytes <= 1024 && (bytes & (bytes - 1)) == 0) return (int)(bytes / 16);
-  return 0;
+  if (bytes < 16 || bytes > 1024 || (bytes & (bytes - 1)) != 0) return 0;
+  return rows * (bytes / 16) <= 0xFFFFFF00ll ? (int)(bytes / 16) : 0;
 }
 
 }  // namespace pkm
@@ -257,7 +258,7 @@ extern "C" int pkm_softmax_fwd(const void* x, int64_t rows, int64_t cols, int dt
   const dim3 grid((unsigned)((rows + 255) / 256));
   hipStream_t st = (hipStream_t)stream;
   const int C = (int)cols;
-  const int lpr = dtype == PKM_DTYPE_F16 ? 0 : sm_vec_lanes(cols, dtype, x, y, y);
+  const int lpr = dtype == PKM_DTYPE_F16 ? 0 : sm_vec_lanes(rows, cols, dtype, x, y, y);
   if (lpr == 0 && sm_wave_path(cols, dtype)) {
     hipLaunchKernelGGL(softmax_fwd_wave_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, x, rows,
                        (int)cols, dtype, y);
@@ -305,7 +306,7 @@ extern "C" int pkm_softmax_bwd(const void* dy, const void* x, int64_t rows, int6
   const dim3 grid((unsigned)((rows + 255) / 256));
   hipStream_t st = (hipStream_t)stream;
   const int C = (int)cols;
-  const int lpr = dtype == PKM_DTYPE_F16 ? 0 : sm_vec_lanes(cols, dtype, dy, x, dx);
+  const int lpr = dtype == PKM_DTYPE_F16 ? 0 : sm_vec_lanes(rows, cols, dtype, dy, x, dx);
   if (lpr == 0 && sm_wave_path(cols, dtype)) {
     hipLaunchKernelGGL(softmax_bwd_wave_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, dy, x, rows,
                        (int)cols, dtype, dx);

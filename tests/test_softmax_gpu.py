@@ -99,3 +99,22 @@ def test_gradient_relative_to_its_terms(device, dtype, shape):
     floor = 2.0**-24 if dtype == torch.float16 else 0.0  # its smallest subnormal
     assert ((dx.double() - expect).abs() <= eps * terms + floor).all()
     assert ((y.double() - p).abs() <= eps * p + floor).all()
+
+
+def test_more_rows_than_a_grid_of_lane_groups(device):
+    """2^28 + 3 rows of 64 float32 (64 GiB): 16 lanes a row would be more
+    threads than a grid holds, so a lane takes a row. Equal scores: 1 / 64."""
+    if torch.cuda.mem_get_info(device)[0] < 160 << 30:
+        pytest.skip("needs 160 GiB of device memory")
+    rows = (1 << 28) + 3
+    x = torch.zeros((rows, 64), device=device)
+    marked = torch.tensor([0, (1 << 28) - 1, 1 << 28, rows - 1], device=device)
+    x[marked] = torch.arange(64, dtype=torch.float32, device=device) / 8
+    y = torch.empty_like(x)
+    _lib.call("pkm_softmax_fwd", _lib.ptr(x), rows, 64, _lib.dtype_code(x), _lib.ptr(y), _lib.stream_of(x.device))
+    assert_rel_close(y[marked], torch.softmax(x[marked].double(), -1), 1e-6, "marked rows")
+    y[marked] = 2.0**-6
+    for a in range(0, rows, 1 << 26):
+        assert bool((y[a:a + (1 << 26)] == 2.0**-6).all()), f"rows from {a}"
+    del x, y
+    torch.cuda.empty_cache()
