@@ -41,16 +41,14 @@ __global__ __launch_bounds__(256) void idw_finish_kernel(const float* __restrict
 }
 #pragma clang fp contract(on)
 
-// 16 lanes a row.
+// 16 lanes a row, the grid's workgroups over all rows.
 __global__ __launch_bounds__(256) void row_sumsq_kernel(const float* __restrict__ x, int64_t B, int64_t T, int dim,
                                                         int row_major, float* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
   const int gl = threadIdx.x & 15;
-  const bool valid = i < B * T;
-  const int64_t b = i / T, t = i - b * T;
-  float a = 0.f;
-  if (valid) {
+  for (int64_t i = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4); i < B * T; i += (int64_t)gridDim.x * 16) {
+    const int64_t b = i / T, t = i - b * T;
     const float* row = x + idw_row(b, t, B, T, dim, row_major);
+    float a = 0.f;
     for (int c = 4 * gl; c < dim; c += 64) {
       const float4 v = *(const float4*)(row + c);
       a = __builtin_fmaf(v.x, v.x, a);
@@ -58,9 +56,9 @@ __global__ __launch_bounds__(256) void row_sumsq_kernel(const float* __restrict_
       a = __builtin_fmaf(v.z, v.z, a);
       a = __builtin_fmaf(v.w, v.w, a);
     }
+    a = group_sum<16>(a);
+    if (gl == 0) out[i] = a;
   }
-  a = group_sum<16>(a);
-  if (valid && gl == 0) out[i] = a;
 }
 
 static int idw_check(const char* what, int64_t batches, int64_t rows, int64_t dim) {
@@ -97,8 +95,8 @@ extern "C" int pkm_row_sumsq(const float* x, int64_t batches, int64_t rows, int6
   if (batches * rows == 0) return PKM_OK;
   PKM_REQUIRE(x && out, PKM_ERR_INVALID_ARGUMENT, "pkm_row_sumsq: null pointer");
   PKM_REQUIRE((uintptr_t)x % 16 == 0, PKM_ERR_INVALID_ARGUMENT, "pkm_row_sumsq: x must be 16-byte aligned");
-  PKM_REQUIRE(batches * rows <= (int64_t)16 * 0x7FFFFFFF, PKM_ERR_INVALID_ARGUMENT, "pkm_row_sumsq: too many rows");
-  hipLaunchKernelGGL(row_sumsq_kernel, dim3((unsigned)((batches * rows + 15) / 16)), dim3(256), 0, (hipStream_t)stream,
-                     x, batches, rows, (int)dim, row_major, out);
+  const int64_t blocks = (batches * rows + 15) / 16;
+  hipLaunchKernelGGL(row_sumsq_kernel, dim3((unsigned)(blocks < (1 << 20) ? blocks : 1 << 20)), dim3(256), 0,
+                     (hipStream_t)stream, x, batches, rows, (int)dim, row_major, out);
   return pkm_check_launch("pkm_row_sumsq");
 }

@@ -49,3 +49,16 @@ def test_long_and_empty_rows(device):
     e = x.transpose(0, 1).double().square().sum(-1)
     assert ((q.double() - e).abs() <= e * dim / 16 * 2.0**-24).all()  # 16 chains a row
     assert torch.equal(pk._row_sumsq(x[..., :0].contiguous(), True), torch.zeros((B, T), device=device))
+
+
+@pytest.mark.parametrize("B,T,row_major", [(2, (1 << 23) + 5, True), (1, (1 << 28) + 3, False)])
+def test_sumsq_of_more_rows_than_a_grid(device, B, T, row_major):
+    """Rows past one round of the grid, and past the 2^32 threads that 16 lanes
+    for each row would be. Whole numbers: exact sums."""
+    shape = (T, B, 4) if row_major else (B, T, 4)
+    x = torch.randint(-8, 9, shape, device=device, dtype=torch.int8).float()
+    q = pk._row_sumsq(x, row_major)
+    expect = (x * x).sum(-1)
+    assert torch.equal(q, expect.t() if row_major else expect)
+    del x, q, expect
+    torch.cuda.empty_cache()
