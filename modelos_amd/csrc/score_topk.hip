@@ -1601,7 +1601,8 @@ __host__ inline size_t lds_bytes(int half) {
 // us by 8 lanes, 32.8 by 32; knn 8, 5000 rows of 128 keys 25.1 and 26.6), and to
 // 8192 for knn > 32 (knn 64, 4096 rows 75 -> 63 us, 8192 rows 102 -> 95).
 static int cartesian_lanes(int64_t rows, int knn) {
-  if (knn > 32) return rows <= 8192 ? 32 : 16;
+  // (2^28 rows of 16 lanes are more threads than a grid holds)
+  if (knn > 32) return rows <= 8192 ? 32 : rows < ((int64_t)1 << 28) - 64 ? 16 : 8;
   return rows <= 4096 ? 32 : 8;
 }
 __host__ inline size_t cartesian_lds_bytes(int knn, int lpr) {

@@ -238,3 +238,26 @@ def test_few_token_tiles_agree(device, dtype, score, half, knn):
         few = score_topk(q[:tokens].to(device), k.to(device), H, knn, score, sub_outputs=True)
         for a, b in zip(few, many):
             assert torch.equal(a, b[: a.shape[0]]), f"tokens {tokens}"
+
+
+def test_more_rows_than_a_grid_of_wide_cartesian_rows(device):
+    """2^28 + 3 rows of knn 33: 16 lanes a row in the cartesian step would be
+    more threads than a grid holds, so 8 take it. The same 97 tokens over and
+    over, whose outputs a short call gives."""
+    if torch.cuda.mem_get_info(device)[0] < 190 << 30:
+        pytest.skip("needs 190 GiB of device memory")
+    T, n, half, knn = (1 << 28) + 3, 64, 32, 33
+    g = gen(500)
+    few = torch.randn((97, 1, 2 * half), generator=g).to(torch.bfloat16).to(device)
+    k = (torch.randn((2 * n, half), generator=g) * half**-0.5).to(torch.bfloat16).to(device)
+    s0, i0 = score_topk(few, k, 1, knn, "dot")[:2]
+    q = few.repeat((T + 96) // 97, 1, 1)[:T]
+    scores, idx = score_topk(q, k, 1, knn, "dot")[:2]
+    del q
+    step = 97 << 17
+    s0, i0 = s0.repeat(step // 97, 1), i0.repeat(step // 97, 1)
+    for a in range(0, T, step):
+        m = min(step, T - a)
+        assert torch.equal(scores[a:a + m], s0[:m]) and torch.equal(idx[a:a + m], i0[:m]), f"rows from {a}"
+    del scores, idx, s0, i0
+    torch.cuda.empty_cache()
