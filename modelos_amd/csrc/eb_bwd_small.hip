@@ -181,41 +181,87 @@ __device__ __forceinline__ void store_grad_row(TW* row, int64_t col0, float* acc
 }
 
 // Chunk c of kHeavyT sorted lookups: the partial sums of the rows of more than
-// kHeavyT lookups in it, by one lane group.
-template <typename TW, typename TG, int LPG, int VPL>
-__device__ __forceinline__ void sparse_heavy_chunk(uint32_t c, const TW* __restrict__ W, int64_t D,
-                                                   const void* __restrict__ psw, int pdt, const TG* __restrict__ g,
-                                                   uint32_t L32, const uint32_t* __restrict__ skeys,
+// kHeavyT lookups in it, by a lane group; or, of rows of 64 VPL SPLIT vectors, its
+// share `part` of the columns: the psw-gradients' parts then meet in `dots`
+// [SPLIT][kHeavyT] (LDS), for add_chunk_dots.
+template <typename TW, typename TG, int LPG, int VPL, int SPLIT = 1>
+__device__ __forceinline__ void sparse_heavy_chunk(uint32_t c, int part, float* dots, const TW* __restrict__ W,
+                                                   int64_t D, const void* __restrict__ psw, int pdt,
+                                                   const TG* __restrict__ g, uint32_t L32,
+                                                   const uint32_t* __restrict__ skeys,
                                                    const uint32_t* __restrict__ svals, uint32_t nv, int glane,
-                                                   float* __restrict__ partials, void* __restrict__ gpsw) {
+                                                   float* __restrict__ partials, void* __restrict__ gpsw,
+                                                   uint32_t* seg) {
   constexpr int EPV = VecTraits<TW>::EPV;
   constexpr int NE = VPL * EPV;
-  const int64_t col0 = (int64_t)glane * EPV;
+  const int64_t col0 = (int64_t)part * VPL * LPG * EPV + (int64_t)glane * EPV;
   const bool want_dot = gpsw != nullptr;
   const uint32_t i_beg = c * kHeavyT;
+  seg[0] = seg[1] = seg[2] = seg[3] = 0;  // the rows' ranges in the chunk
   if (i_beg >= nv) return;
   const uint32_t i_end = i_beg + kHeavyT < nv ? i_beg + kHeavyT : nv;
   const uint32_t cand[2] = {skeys[i_beg], skeys[i_end - 1]};
+  const uint32_t before = i_beg > 0 ? skeys[i_beg - 1] : 0xFFFFFFFFu, after = i_end < nv ? skeys[i_end] : 0xFFFFFFFFu;
 #pragma unroll 1
   for (int t = 0; t < 2; ++t) {
     const uint32_t r = cand[t];
     if (t == 1 && r == cand[0]) break;
-    if (!((i_beg > 0 && skeys[i_beg - 1] == r) || (i_end < nv && skeys[i_end] == r))) continue;  // inside the chunk
-    uint32_t rb, re;
-    run_of(skeys, nv, r, &rb, &re);
-    if (re - rb <= (uint32_t)kHeavyT) continue;
-    const uint32_t s_beg = rb > i_beg ? rb : i_beg, s_end = re < i_end ? re : i_end;
+    if (before != r && after != r) continue;  // inside the chunk
+    uint32_t s_beg = i_beg, s_end = i_end;
+    if (cand[0] != cand[1]) {  // the row's first or last place in the chunk
+      const uint32_t key = r + (t == 0 ? 1u : 0u);
+      uint32_t lo = i_beg, hi = i_end;
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (skeys[mid] < key)
+          lo = mid + 1;
+        else
+          hi = mid;
+      }
+      // more than kHeavyT lookups: the row is also kHeavyT places before its last one, or past its first
+      if (t == 0) {
+        s_end = lo;
+        if (s_end <= (uint32_t)kHeavyT || skeys[s_end - 1 - kHeavyT] != r) continue;
+      } else {
+        s_beg = lo;
+        if (nv - s_beg <= (uint32_t)kHeavyT || skeys[s_beg + kHeavyT] != r) continue;
+      }
+    } else if (i_end - i_beg < (uint32_t)kHeavyT && (i_beg == 0 || skeys[i_end - 1 - kHeavyT] != r)) {
+      continue;  // (the last, shorter chunk)
+    }
+    if (t == 0) {
+      seg[0] = s_beg;
+      seg[1] = s_end;
+    } else {
+      seg[2] = s_beg;
+      seg[3] = s_end;
+    }
     float wv[NE], acc[NE];
     if (want_dot) load_row_f32<TW, LPG, VPL>(W + (int64_t)r * D, col0, wv);
 #pragma unroll
     for (int e = 0; e < NE; ++e) acc[e] = 0.f;
-    reduce_occurrences<TW, TG, LPG, VPL>(s_beg, s_end, svals, psw, pdt, g, D, L32, col0, glane, wv, want_dot, gpsw,
-                                         acc);
-    float* prow = partials + (2 * (int64_t)c + (rb > i_beg ? 1 : 0)) * D + col0;
+    reduce_occurrences<TW, TG, LPG, VPL>(s_beg, s_end, svals, psw, pdt, g, D, L32, col0, glane, wv, want_dot, gpsw, acc,
+                                         SPLIT > 1 ? dots + part * kHeavyT - (int64_t)i_beg : nullptr);
+    float* prow = partials + (2 * (int64_t)c + (s_beg > i_beg ? 1 : 0)) * D + col0;
 #pragma unroll
     for (int v = 0; v < VPL; ++v)
 #pragma unroll
       for (int h = 0; h < EPV; h += 4) st16(prow + v * LPG * EPV + h, VecTraits<float>::pack(acc + v * EPV + h));
+  }
+}
+
+// The psw-gradients of chunk c's ranges `seg`, their parts added in order.
+template <int SPLIT>
+__device__ __forceinline__ void add_chunk_dots(uint32_t c, const uint32_t* seg, const float* dots,
+                                               const uint32_t* __restrict__ svals, int pdt, int thread,
+                                               void* __restrict__ gpsw) {
+  for (int i = thread; i < kHeavyT; i += 64 * SPLIT) {
+    const uint32_t p = c * kHeavyT + (uint32_t)i;
+    if (!((p >= seg[0] && p < seg[1]) || (p >= seg[2] && p < seg[3]))) continue;
+    float d = dots[i];
+#pragma unroll
+    for (int k = 1; k < SPLIT; ++k) d += dots[k * kHeavyT + i];
+    store_scalar(gpsw, pdt, svals[p], d);
   }
 }
 
@@ -253,8 +299,10 @@ __global__ __launch_bounds__(256) void sparse_narrow_kernel(const TW* __restrict
   const uint32_t j = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * GPW + lane / LPG;
   const uint32_t nv = *nvalid;
   if (j >= N) {
+    uint32_t seg[4];
     if (j < N + nchunks)
-      sparse_heavy_chunk<TW, TG, LPG, VPL>(j - N, W, D, psw, pdt, g, L32, skeys, svals, nv, glane, partials, gpsw);
+      sparse_heavy_chunk<TW, TG, LPG, VPL>(j - N, 0, nullptr, W, D, psw, pdt, g, L32, skeys, svals, nv, glane, partials,
+                                           gpsw, seg);
     return;
   }
   const bool want_dot = gpsw != nullptr;
@@ -279,7 +327,11 @@ __global__ __launch_bounds__(256) void sparse_narrow_kernel(const TW* __restrict
 // lookups [win j, win (j + 1)), streamed in position order, U lookups' rows
 // in flight: the 64 lookups from the window's start are held one per lane (one
 // coalesced read each of row, position and weight), a run past them (at most
-// kHeavyT lookups) goes on in steps of its own. Wave nwin + c: heavy chunk c.
+// kHeavyT lookups) goes on in steps of its own. The last workgroups take the
+// heavy chunks: of rows of several vectors a lane up to 4 waves a chunk, each a
+// share of the columns, whose loads of all 256 lookups would else hang on one
+// wave's 1 to 4 in flight (1024 x 10 lookups in rows of 300, 4096 x 8 KB bf16 234
+// -> 145 us, in rows of 1000 225 -> 127, 2 KB 103 -> 89).
 // The out-of-range lookups' psw-gradients are zeroed on the way: the sorted
 // ones past nvalid (small_sort), or the list `invalid`.
 // (A wave per lookup pays five dependent reads for each: backward of 262144
@@ -291,9 +343,17 @@ __global__ __launch_bounds__(256) void sparse_narrow_kernel(const TW* __restrict
 constexpr int kWin = 16;
 constexpr int kWinFew = 4;
 constexpr int64_t kWinFewLookups = 163840;
+template <int VPL>
+constexpr int kChunkSplit = VPL < 4 ? VPL : 4;  // waves per heavy chunk
+
+// (Waves per SIMD: what the row's registers leave with its loads in flight. Left
+// to itself the compiler trades those for one wave more: 10 x 1000 lookups in rows
+// of 200 of 512 x 8 KB f32 101 -> 113 us.)
+template <typename TW, int VPL>
+constexpr int kRunsWaves = VPL * VecTraits<TW>::EPV >= 32 ? 2 : VPL * VecTraits<TW>::EPV >= 16 ? 3 : 8;
 
 template <typename TW, typename TG, int VPL, bool ACC>
-__global__ __launch_bounds__(256) void sparse_runs_kernel(const TW* __restrict__ W, int64_t D,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, kRunsWaves<TW, VPL>))) void sparse_runs_kernel(const TW* __restrict__ W, int64_t D,
                                                           const void* __restrict__ psw, int pdt,
                                                           const TG* __restrict__ g, uint32_t L32,
                                                           const uint32_t* __restrict__ skeys,
@@ -308,15 +368,30 @@ __global__ __launch_bounds__(256) void sparse_runs_kernel(const TW* __restrict__
   constexpr int NE = VPL * EPV;
   constexpr int NV = GT::NV;
   constexpr int U = VPL * NV >= 8 ? 1 : 8 / (VPL * NV);
+  constexpr int SPLIT = kChunkSplit<VPL>;
+  constexpr uint32_t CPB = 4 / SPLIT;  // chunks per workgroup
+  __shared__ float dots[4][kHeavyT];
   const int lane = threadIdx.x & 63;
-  const uint32_t j = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t nv = *nvalid;
   const uint32_t nwin = (N + win - 1) / win;
-  if (j >= nwin) {
-    if (j - nwin < nchunks)
-      sparse_heavy_chunk<TW, TG, 64, VPL>(j - nwin, W, D, psw, pdt, g, L32, skeys, svals, nv, lane, partials, gpsw);
+  const uint32_t wblocks = (nwin + 3) / 4;
+  if (blockIdx.x >= wblocks) {
+    uint32_t seg[4] = {0, 0, 0, 0};
+    const uint32_t c = (blockIdx.x - wblocks) * CPB + wave / SPLIT;
+    float* const cdots = dots[wave / SPLIT * SPLIT];
+    if (c < nchunks)
+      sparse_heavy_chunk<TW, TG, 64, VPL / SPLIT, SPLIT>(c, (int)(wave % SPLIT), cdots, W, D, psw, pdt, g, L32, skeys,
+                                                         svals, nv, lane, partials, gpsw, seg);
+    if constexpr (SPLIT > 1) {
+      __syncthreads();
+      if (gpsw != nullptr)
+        add_chunk_dots<SPLIT>(c, seg, cdots, svals, pdt, (int)(wave % SPLIT) * 64 + lane, gpsw);
+    }
     return;
   }
+  const uint32_t j = blockIdx.x * 4 + wave;
+  if (j >= nwin) return;
   const bool want_dot = gpsw != nullptr;
   if (invalid != nullptr && want_dot) {  // the out-of-range lookups, listed (count first) by the sort
     const uint32_t n = invalid[0];
@@ -484,14 +559,15 @@ static void launch_sparse(const void* W, int64_t K, int64_t D, const void* psw, 
   KernelSpan span("eb_bwd_rows", st);
   if constexpr (LPG == 64) {
     const int win = N > kWinFewLookups ? kWin : kWinFew;
-    const int64_t waves = (N + win - 1) / win + nchunks;
-    hipLaunchKernelGGL((sparse_runs_kernel<TW, TG, VPL, ACC>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st,
+    const int64_t cpb = 4 / kChunkSplit<VPL>;
+    const int64_t blocks = (nchunks + cpb - 1) / cpb + ((N + win - 1) / win + 3) / 4;
+    hipLaunchKernelGGL((sparse_runs_kernel<TW, TG, VPL, ACC>), dim3((unsigned)blocks), dim3(256), 0, st,
                        (const TW*)W, D, psw, pdt, (const TG*)g, (uint32_t)L, skeys, svals, nvalid, (uint32_t)N,
                        (uint32_t)nchunks, win, invalid, partials, (TW*)gW, gpsw);
   } else {
     static_assert(!ACC, "the accumulating reduction runs on 64-lane rows");
-    hipLaunchKernelGGL((sparse_narrow_kernel<TW, TG, LPG, VPL>), dim3((unsigned)((N + nchunks + GPB - 1) / GPB)),
-                       dim3(256), 0, st, (const TW*)W, D, psw, pdt, (const TG*)g, (uint32_t)L, skeys, svals, nvalid,
+    hipLaunchKernelGGL((sparse_narrow_kernel<TW, TG, LPG, VPL>),
+                       dim3((unsigned)((N + nchunks + GPB - 1) / GPB)), dim3(256), 0, st, (const TW*)W, D, psw, pdt, (const TG*)g, (uint32_t)L, skeys, svals, nvalid,
                        (uint32_t)N, (uint32_t)nchunks, partials, (TW*)gW, gpsw);
   }
   if (nchunks > 0)

@@ -156,10 +156,11 @@ __device__ __forceinline__ bool fill_share(const FillShare& f) {  // true: not o
 // Few lookups, general -> sparse, backward: uniform and Zipf(1.1) lookups, 64 to
 // 2^20 rows of 32 bytes to 8 KB, were faster in each of 1488 cases, 1.03 to 31
 // times (10 x 1000 into 2^9 x 4096 bf16 916 -> 77 us, 64 x 64 into 2^16 x 64 bf16
-// 49 -> 26), also where the lookups are far more than the rows. Lookups that all
-// lie in a few rows are the exception: 1024 x 10 in 34 rows of 300 each, whose rows
-// the general plan reduces on the matrix cores, 8 KB bf16 168 -> 235 us, 4 KB 132
-// -> 161, 2 KB 116 -> 107; 51 rows of 200, 8 KB 260 -> 187.
+// 49 -> 26), also where the lookups are far more than the rows. So are lookups that
+// all lie in a few rows (1024 x 10 in 34 rows of 300, which the general plan
+// reduces on the matrix cores, 8 KB bf16 171 -> 145 us, 4 KB 130 -> 109), except in
+// rows of 512 bytes and less, a lane group each (512 bytes, 10 rows of 1000 123 ->
+// 148, 51 rows of 200 110 -> 121).
 // ---------------------------------------------------------------------------
 constexpr int64_t kSmallLookups = 10240;  // (14 bytes of LDS each in the sort)
 inline bool small_plan(int64_t N) { return N > 0 && N <= kSmallLookups; }

@@ -1025,3 +1025,41 @@ def test_backward_accumulate_unsupported_returns_none(device):
     buf = torch.zeros((K, 1024), device=device, dtype=torch.bfloat16)
     assert eb.eb_backward_into(idd, Wd, pd, gd.float(), buf) is None  # float32 gradient of a bf16 table
     assert torch.count_nonzero(buf) == 0
+
+
+# Rows of more than 256 lookups on the sparse plan, whose chunks several waves
+# share by columns: rows that start, end, start and end at a chunk's edge, cover
+# chunks, two in one chunk, of 255 to 257 lookups, the last chunk short; 1, 2, 4
+# and 8 vectors a lane, and narrow rows. Sums in chunk order: the table gradients
+# are those of the same lookups with the general plan (more than 10240 lookups, the
+# others out of range), bit for bit, where that uses no matrix-core products.
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 256), (torch.float32, 512), (torch.float32, 1024),
+                                     (torch.float32, 2048), (torch.bfloat16, 4096), (torch.bfloat16, 1024),
+                                     (torch.float16, 2048), (torch.bfloat16, 256), (torch.float32, 16)], ids=str)
+@pytest.mark.parametrize("counts", [(256, 257, 255, 300, 212, 513, 100), (10, 246, 512, 600, 400), (1000,),
+                                    (3, 257, 252, 512, 256)], ids=str)
+def test_backward_sparse_plan_heavy_chunks(counts, dtype, D, device):
+    from modelos_amd import embedding_bag as eb
+
+    K, L = 700, 8
+    n = sum(counts)
+    B = -(-n // L)
+    W, _, p, g = eb_inputs(B, L, K, D, dtype, seed=95 + n)
+    gen = torch.Generator().manual_seed(96)
+    flat = torch.full((B * L,), -1)
+    flat[:n] = torch.cat([torch.full((c,), 5 + 3 * i) for i, c in enumerate(counts)])
+    idx = flat[torch.randperm(B * L, generator=gen)].view(B, L)
+    gW, gp = eb.eb_backward(*_dev(idx, W, p, g, device=device))
+    eW, ep = ref.eb_backward(idx, W, p, g)
+    cW, cp = ref.eb_backward(idx, W.abs(), p.abs(), g.abs())
+    assert_rel_close(gW, eW, REL_TOL[dtype], "grad_weight", cond=cW)
+    assert_rel_close(gp, ep, REL_TOL[dtype], "grad_psw", cond=cp)
+    uW, _ = eb.eb_backward(*_dev(idx, W, None, g, device=device))  # no psw-gradients
+    ones = torch.ones_like(p)
+    assert torch.equal(uW, eb.eb_backward(*_dev(idx, W, ones, g, device=device))[0])
+    if dtype != torch.bfloat16:
+        extra = 10241 // L + 1
+        idx2 = torch.cat([idx, torch.full((extra, L), -1)])
+        p2, g2 = torch.cat([p, p.new_zeros((extra, L))]), torch.cat([g, g.new_zeros((extra, D))])
+        big = eb.eb_backward(*_dev(idx2, W, p2, g2, device=device))
+        assert torch.equal(big[0], gW)
